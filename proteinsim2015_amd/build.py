@@ -116,7 +116,7 @@ def build_oracle(verbose: bool = False) -> None:
     sys.path.insert(0, ROOT)
     from oracle.oracle import build_oracle as _b  # test infrastructure
     _b(force=True)
-    if os.path.isdir(REFERENCE):
+    if os.path.isdir(os.path.join(REFERENCE, "ClusteredCore")):
         _run(["make", "-s", "-C", os.path.join(ROOT, "oracle", "ref"), f"REF={REFERENCE}",
               "-j8"], verbose)
 
