@@ -479,6 +479,7 @@ int restore_cp(psim_adjoint *A, int k)
     add_seg(cs, ip, c->id, sizeof(int) * c->n);
     add_seg(cs, ip + c->n, c->cstart, sizeof(int) * (c->ncell + 1));
     int rc = copy_segs(c, cs);
+    if (!rc) rc = eng::pack_positions(c);
     if (rc) return rc;
     c->lagged = false;
     c->time = A->meta[k].time;

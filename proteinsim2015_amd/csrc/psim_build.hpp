@@ -11,7 +11,7 @@
 // sort), which makes every run reproducible bit for bit.
 #pragma once
 
-#include "psim_device.hpp"
+#include "psim_gather.hpp"
 
 namespace psim {
 namespace {
@@ -260,45 +260,9 @@ __global__ __launch_bounds__(256) void k_scatter(int n, const int *key, const in
     }
 }
 
-// Canonical order within a cell = ascending source slot (stable counting
-// sort); gathers the state into the sorted arrays.
-__global__ void k_move(int n, const int *__restrict__ perm, const int *__restrict__ key,
-                       const int *__restrict__ cstart, const double *__restrict__ npos,
-                       const double *__restrict__ npos0, const double *__restrict__ nfrc,
-                       const double *__restrict__ nmem, const int *__restrict__ nid,
-                       double *__restrict__ pos, double *__restrict__ pos0,
-                       double *__restrict__ frc, double *__restrict__ mem,
-                       int *__restrict__ id)
-{
-    // the source and destination arrays are distinct buffers (restrict lets
-    // all twelve gathers issue before the first store)
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int s = perm[t];
-    const int c = key[s];
-    const int b = cstart[c], e = cstart[c + 1];
-    // four independent loads per round (the count is latency-bound otherwise)
-    int rank = 0;
-    int u = b;
-    for (; u + 4 <= e; u += 4) {
-        const int p0 = perm[u], p1 = perm[u + 1], p2 = perm[u + 2], p3 = perm[u + 3];
-        rank += (p0 < s) + (p1 < s) + (p2 < s) + (p3 < s);
-    }
-    for (; u < e; ++u) rank += (perm[u] < s);
-    const int dst = b + rank;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        pos[d * n + dst] = npos[d * n + s];
-        pos0[d * n + dst] = npos0[d * n + s];
-        frc[d * n + dst] = nfrc[d * n + s];
-        mem[d * n + dst] = nmem[d * n + s];
-    }
-    id[dst] = nid[s];
-}
-
-
-// As k_move, but only the positions and the original ids are gathered into
-// the new order; prev[dst] records the slot each particle came from, so the
+// Canonical order within a cell = ascending source slot (a stable counting
+// sort).  Only the positions and the original ids are gathered into the new
+// order; prev[dst] records the slot each particle came from, so the
 // integrator reads the previous positions, forces and memory of the last
 // step where it wrote them (at prev[s]) instead of every array moving every
 // step.
@@ -320,31 +284,47 @@ constexpr int kMoveIlp = PSIM_MOVE_ILP;
 // below this many particles the grid is too small to give up lanes for
 // interleaving (one particle per lane)
 constexpr int kMoveIlpMin = 1 << 20;
-template <int U>
+// 1 / L of the box that slot t's particle lives in: one box for all; NoBox
+// where the pair kernel reads no box fractions.
+struct OneBox {
+    static constexpr bool kPack = true;
+    double inv_L;
+    __device__ double operator()(int) const { return inv_L; }
+};
+struct NoBox {
+    static constexpr bool kPack = false;
+    __device__ double operator()(int) const { return 0.0; }
+};
+// Box::kPack: the new positions' box fractions and cells are written to upos
+// too (the thread-per-particle kernels' cull).
+template <int U, class Box>
 __global__ __launch_bounds__(256) void k_move_lagged(
     int n, const int *__restrict__ perm, const int *__restrict__ key,
     const int *__restrict__ cstart, const double *__restrict__ npos,
     const int *__restrict__ id_in, double *__restrict__ pos, int *__restrict__ id_out,
-    int *__restrict__ prev, StepCtl *ctl, double *__restrict__ pos2 = nullptr,
-    int *__restrict__ id2 = nullptr, int *__restrict__ inv2 = nullptr)
+    int *__restrict__ prev, StepCtl *ctl, uint4 *__restrict__ upos, Box box,
+    double *__restrict__ pos2 = nullptr, int *__restrict__ id2 = nullptr,
+    int *__restrict__ inv2 = nullptr)
 {
     const int t0 = blockIdx.x * (blockDim.x * U) + threadIdx.x;
     if (ctl && t0 == 0) ctl_advance(ctl);
     if (t0 >= n) return;
-    int s[U], b[U], len[U], rank[U];
+    int s[U], c[U], b[U], len[U], rank[U];
+    double inv_L[U];
     bool ok[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int t = t0 + u * (int)blockDim.x;
         ok[u] = t < n;
         s[u] = perm[ok[u] ? t : t0];   // a missing slot repeats the first
+        if (Box::kPack) inv_L[u] = box(ok[u] ? t : t0);   // the box of the slot's cell
     }
     int most = 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const int c = key[s[u]];
-        b[u] = cstart[c];
-        len[u] = cstart[c + 1] - b[u];
+        c[u] = key[s[u]];
+        b[u] = cstart[c[u]];
+        len[u] = cstart[c[u] + 1] - b[u];
         rank[u] = 0;
         most = max(most, len[u]);
     }
@@ -375,6 +355,7 @@ __global__ __launch_bounds__(256) void k_move_lagged(
             pos[d * n + dst] = x[u][d];
             if (pos2) pos2[d * n + dst] = x[u][d];
         }
+        if (Box::kPack) upos[dst] = pack_position(x[u][0], x[u][1], x[u][2], c[u], inv_L[u]);
         id_out[dst] = o[u];
         if (id2) id2[dst] = o[u];
         if (inv2) inv2[o[u]] = dst;

@@ -28,6 +28,7 @@ struct psim_ctx {
     psim::Geo geo;
     psim::Pot pot;
     psim::GB gb;
+    psim::Cull cull;   // derived from geo and pot
     int n = 0, ncell = 0, nscan = 0;
     bool dense = false;   // cell-per-workgroup pair kernel (else thread per particle)
     bool brick = false;   // brick-per-workgroup pair kernel (sparse systems)
@@ -37,6 +38,8 @@ struct psim_ctx {
     double *pos = nullptr, *pos0 = nullptr, *frc = nullptr, *mem = nullptr;
     double *npos = nullptr, *npos0 = nullptr, *nfrc = nullptr, *nmem = nullptr;
     double *vel = nullptr, *fout = nullptr;
+    uint4 *upos = nullptr;   // box fractions and cells of pos, in its slot order
+                             // (thread-per-particle path only)
     int *id = nullptr, *nid = nullptr, *key = nullptr, *arank = nullptr, *perm = nullptr;
     // pos0 / frc / mem stay in the slot order of the last step: pos0 the
     // positions that step started from (not yet re-imaged), frc and mem what
@@ -57,6 +60,7 @@ struct psim_ctx {
     double *noise = nullptr;
     size_t noise_cap = 0;
     double *tsorted = nullptr;
+    uint4 *tupos = nullptr;
     int *thi = nullptr, *tcse = nullptr;
     int *st_count = nullptr;                 // neighbour-set statistics
     unsigned long long *st_hash = nullptr;
@@ -127,6 +131,9 @@ int launch_build(psim_ctx *c);
 // gather lagged pos0 / frc / mem into the current slot order (no-op when
 // they are in it already)
 int settle(psim_ctx *c);
+// upos of the positions the context now holds (after something other than
+// the cell rebuild has written them)
+int pack_positions(psim_ctx *c);
 // nsteps of system::run with the context's step bookkeeping
 int run_steps(psim_ctx *c, int nsteps, const double *d_noise);
 int read_error(psim_ctx *c, int *code, int *i, int *j);

@@ -13,8 +13,7 @@
 namespace psim {
 
 constexpr int kBlock = 256;        // threads per block of the pair kernels
-constexpr int kHitCap = 32;        // per-lane capacity of the LDS hit list
-constexpr unsigned kIdxBits = 26;  // slot index bits in a hit-list entry
+constexpr unsigned kIdxBits = 26;  // slot index bits in a pair-list entry
 constexpr unsigned kIdxMask = (1u << kIdxBits) - 1u;
 
 enum { F_CAL = 1, F_LJ = 2, F_AO = 4 };
@@ -33,6 +32,15 @@ struct Geo {
     int c0;           // offset of this system's cells in the cell-index space
                       // (0 for one system; replicas of an ensemble are
                       // stacked, each owning S^3 consecutive cells)
+};
+
+// What the wave-wide gather (psim_gather.hpp) needs beside Geo and Pot.
+struct Cull {
+    double inv_L;     // 1 / L
+    double inv_S2;    // 1 / S^2
+    float inv_S;      // 1 / S
+    float ucut2;      // Pot::rc2_hi in box fractions, (2^-32 box)^2, with the
+                      // cull's margin
 };
 
 // Pair-force constants (LJPotential.cpp:34-55, AOPotential.cpp:40-55).

@@ -51,7 +51,11 @@ namespace {
 using eng::blocks_for;
 using eng::dalloc;
 
-void fill_constants(psim_ctx *c) { make_constants(c->prm, c->geo, c->pot, c->gb); }
+void fill_constants(psim_ctx *c)
+{
+    make_constants(c->prm, c->geo, c->pot, c->gb);
+    c->cull = make_cull(c->geo, c->pot);
+}
 
 hipEvent_t take_event(psim_ctx *c, size_t *idx)
 {
@@ -111,14 +115,20 @@ int launch_build(psim_ctx *c, StepCtl *advance)
     // integrator, not after it); the positions this step started from become
     // pos0, and they, the forces and the memory stay where this step had or
     // wrote them (old order): the next step reads them through prev
-    if (n >= kMoveIlpMin)
-        k_move_lagged<kMoveIlp><<<blocks_for(n, 256 * kMoveIlp), 256, 0, st>>>(
-            n, c->perm, c->key, c->cstart, c->npos, c->id, c->pos0, c->nid, c->prev, advance,
-            c->rec.pos, c->rec.id, c->rec.inv);
+    auto move = [&](auto box) {
+        if (n >= kMoveIlpMin)
+            k_move_lagged<kMoveIlp><<<blocks_for(n, 256 * kMoveIlp), 256, 0, st>>>(
+                n, c->perm, c->key, c->cstart, c->npos, c->id, c->pos0, c->nid, c->prev, advance,
+                c->upos, box, c->rec.pos, c->rec.id, c->rec.inv);
+        else
+            k_move_lagged<1><<<blocks_for(n, 256), 256, 0, st>>>(
+                n, c->perm, c->key, c->cstart, c->npos, c->id, c->pos0, c->nid, c->prev, advance,
+                c->upos, box, c->rec.pos, c->rec.id, c->rec.inv);
+    };
+    if (c->upos)
+        move(OneBox{c->cull.inv_L});
     else
-        k_move_lagged<1><<<blocks_for(n, 256), 256, 0, st>>>(
-            n, c->perm, c->key, c->cstart, c->npos, c->id, c->pos0, c->nid, c->prev, advance,
-            c->rec.pos, c->rec.id, c->rec.inv);
+        move(NoBox{});
     CK(hipGetLastError());
     std::swap(c->id, c->nid);
     std::swap(c->pos, c->pos0);
@@ -142,6 +152,25 @@ int settle(psim_ctx *c)
     CK(hipMemcpyAsync(c->frc, c->nfrc, b, hipMemcpyDeviceToDevice, c->stream));
     CK(hipMemcpyAsync(c->mem, c->nmem, b, hipMemcpyDeviceToDevice, c->stream));
     c->lagged = false;
+    return 0;
+}
+
+__global__ void k_pack(Geo g, double inv_L, const double *pos, uint4 *upos)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= g.n) return;
+    const double x = pos[s], y = pos[g.n + s], z = pos[2 * g.n + s];
+    upos[s] = pack_position(x, y, z,
+                            cell_1d(x, g.cell, g.S) + g.S * cell_1d(y, g.cell, g.S)
+                                + g.S2 * cell_1d(z, g.cell, g.S), inv_L);
+}
+
+int pack_positions(psim_ctx *c)
+{
+    if (!c->upos) return 0;
+    k_pack<<<blocks_for(c->n, 256), 256, 0, c->stream>>>(c->geo, c->cull.inv_L, c->pos,
+                                                            c->upos);
+    CK(hipGetLastError());
     return 0;
 }
 
@@ -183,10 +212,10 @@ void launch_step_mask(psim_ctx *c, const StepArgs &a)
         // that every CU gets work
         k_step<MASK, 64, kSmallSplit>
             <<<xcd_grid(blocks_for((long long)c->n * kSmallSplit, 64)), 64, 0, c->stream>>>(
-                c->geo, c->pot, c->gb, c->prm.radius, a);
+                c->geo, c->pot, c->cull, c->gb, c->prm.radius, a);
     } else {
         k_step<MASK, kBlock><<<xcd_grid(blocks_for(c->n, kBlock)), kBlock, 0, c->stream>>>(
-            c->geo, c->pot, c->gb, c->prm.radius, a);
+            c->geo, c->pot, c->cull, c->gb, c->prm.radius, a);
     }
 }
 
@@ -224,7 +253,8 @@ void launch_forces_mask(psim_ctx *c)
             c->err);
     } else {
         k_forces<MASK><<<xcd_grid(blocks_for(c->n, kBlock)), kBlock, 0, c->stream>>>(
-            c->geo, c->pot, c->prm.radius, c->pos, c->id, c->cstart, c->fout, c->err);
+            c->geo, c->pot, c->cull, c->prm.radius, c->pos, c->upos, c->id, c->cstart, c->fout,
+            c->err);
     }
 }
 
@@ -247,18 +277,28 @@ void launch_stats(psim_ctx *c, NbrStatsOut so)
     } else if (c->n < kSmallSystem) {
         k_stats<64, kSmallSplit>
             <<<xcd_grid(blocks_for((long long)c->n * kSmallSplit, 64)), 64, 0, c->stream>>>(
-                c->geo, c->pot, c->prm.radius, c->pos, c->id, c->cstart, so);
+                c->geo, c->pot, c->cull, c->prm.radius, c->pos, c->upos, c->id, c->cstart, so);
     } else {
         k_stats<kBlock, 1><<<xcd_grid(blocks_for(c->n, kBlock)), kBlock, 0, c->stream>>>(
-            c->geo, c->pot, c->prm.radius, c->pos, c->id, c->cstart, so);
+            c->geo, c->pot, c->cull, c->prm.radius, c->pos, c->upos, c->id, c->cstart, so);
     }
 }
 
 template <int MASK>
 void launch_table_mask(psim_ctx *c)
 {
-    k_forces_table<MASK><<<blocks_for(c->n, kBlock), kBlock, 0, c->stream>>>(
-        c->geo, c->pot, c->tsorted, c->thi, c->tcse, c->fout, c->err);
+    k_pack_table<<<blocks_for(c->n, 256), 256, 0, c->stream>>>(c->geo, c->cull.inv_L, c->tsorted,
+                                                              c->tupos);
+    if (c->n < kSmallSystem)
+        k_forces_table<MASK, 64, kSmallSplit>
+            <<<xcd_grid(blocks_for((long long)c->n * kSmallSplit, 64)), 64, 0, c->stream>>>(
+                c->geo, c->pot, c->cull, c->tsorted, c->tupos, c->thi, c->tcse, c->fout,
+                c->err);
+    else
+        k_forces_table<MASK, kBlock, 1>
+            <<<xcd_grid(blocks_for(c->n, kBlock)), kBlock, 0, c->stream>>>(
+                c->geo, c->pot, c->cull, c->tsorted, c->tupos, c->thi, c->tcse, c->fout,
+                c->err);
 }
 
 // The step arguments of the context's current buffers.  ctl: the kernels
@@ -268,7 +308,7 @@ StepArgs step_args(psim_ctx *c, const double *noise, const StepCtl *ctl)
 {
     StepArgs a{};
     a.pos = c->pos; a.pos0 = c->pos0; a.frc = c->frc; a.mem = c->mem;
-    a.id = c->id; a.cstart = c->cstart;
+    a.upos = c->upos; a.id = c->id; a.cstart = c->cstart;
     a.prev = c->lagged ? c->prev : nullptr;
     a.x0_raw = c->lagged ? 1 : 0;
     a.npos = c->npos; a.npos0 = c->npos0; a.nfrc = c->nfrc; a.nmem = c->nmem;
@@ -543,6 +583,7 @@ int set_state(psim_ctx *c, const double *pos, const double *pos0, const double *
 
 int launch_build(psim_ctx *c) { return ::launch_build(c, nullptr); }
 int settle(psim_ctx *c) { return ::settle(c); }
+int pack_positions(psim_ctx *c) { return ::pack_positions(c); }
 int run_steps(psim_ctx *c, int nsteps, const double *d_noise)
 {
     return ::run_steps(c, nsteps, d_noise);
@@ -608,6 +649,7 @@ int psim_gpu_create(const psim_params *params, psim_ctx **out)
     if (!rc) rc = dalloc(&c->nmem, n3);
     if (!rc) rc = dalloc(&c->vel, n3);
     if (!rc) rc = dalloc(&c->fout, n3);
+    if (!rc && !c->dense && !c->brick) rc = dalloc(&c->upos, c->n);
     if (!rc) rc = dalloc(&c->id, c->n);
     if (!rc) rc = dalloc(&c->nid, c->n);
     if (!rc) rc = dalloc(&c->key, c->n);
@@ -667,7 +709,7 @@ void psim_gpu_destroy(psim_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
     void *bufs[] = {c->pos, c->pos0, c->frc, c->mem, c->npos, c->npos0, c->nfrc,
-                    c->nmem, c->vel, c->fout, c->id, c->nid, c->key, c->arank,
+                    c->nmem, c->vel, c->fout, c->upos, c->tupos, c->id, c->nid, c->key, c->arank,
                     c->perm, c->prev, c->ctl, c->count, c->cstart, c->bsum, c->err, c->noise,
                     c->tsorted, c->thi, c->tcse, c->st_count, c->st_hash, c->pbc,
                     c->track0, c->hg.key,
@@ -810,6 +852,7 @@ int psim_gpu_force_table(psim_ctx *c, const double *sorted4, const int *hash_ind
     int rc = 0;
     if (!c->tsorted) {
         if (!rc) rc = dalloc(&c->tsorted, 4 * (size_t)n);
+        if (!rc) rc = dalloc(&c->tupos, n);
         if (!rc) rc = dalloc(&c->thi, 2 * (size_t)n);
         if (!rc) rc = dalloc(&c->tcse, 2 * (size_t)c->ncell);
         if (rc) return rc;

@@ -44,8 +44,23 @@ namespace {
 struct RepGeo {
     Geo g;       // g.n = Ntot (array stride), g.c0 = first cell of the replica
     Pot p;
+    Cull q;
     double radius;
     BrickGeo bg;   // the replica's bricks (brick kernel)
+};
+
+// 1 / L of the box of slot t (k_move_lagged): rep_of names the replica of
+// slots 0, 256, 512, ...; the replica of t is that one or a later one.
+struct ReplicaBox {
+    static constexpr bool kPack = true;
+    const int *rep_of, *p0;
+    const RepGeo *reps;
+    __device__ double operator()(int t) const
+    {
+        int r = rep_of[t >> 8];
+        while (p0[r + 1] <= t) ++r;
+        return reps[r].q.inv_L;
+    }
 };
 
 // replica owning original id o: last r with p0[r] <= o
@@ -59,47 +74,45 @@ __device__ __forceinline__ int replica_of(const int *__restrict__ p0, int nrep, 
     return lo;
 }
 
-// Thread-per-particle pair forces for the replicas rmap[0..nrep): workgroup
-// `it` of the launch covers slots p0[r] + (it - blk0[l]) BLOCK .. of replica
-// r = rmap[l] (blk0 = prefix of those replicas' workgroup counts; the
-// replicas of one occupancy class, see EnsClass), so a workgroup never spans
-// two replicas and
-// the replica's geometry and constants are the same for every lane (scalar
-// loads, no per-lane replica search).  The forces go to nfrc, where the
-// integrator (k_ens_integ, the same launch shape) reads them: as two
-// kernels the 5.25 M-particle ensemble step takes 0.927 ms against 0.945
-// with the integrator in this kernel's epilogue.
+// A workgroup's replica and its first slot.  The thread-per-particle kernels
+// read it from a table made with the launch shape: one load in place of a
+// binary search over the replicas, ten dependent loads at the start of every
+// workgroup.
+struct WorkGroup {
+    int r, s0;
+};
+
+// Thread-per-particle pair forces: workgroup `it` of the launch covers slots
+// wg[it].s0 .. + BLOCK of replica wg[it].r (the replicas of one occupancy
+// class, see EnsClass), so a workgroup never spans two replicas and the
+// replica's geometry and constants are the same for every lane (scalar
+// loads).  The forces go to nfrc, where the integrator (k_ens_integ) reads
+// them: with the integrator in this kernel's epilogue the 5.25 M-particle
+// ensemble step took 0.945 ms against 0.927.
 template <int MASK, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_ens_step(const RepGeo *__restrict__ reps,
-                                                    const int *__restrict__ p0,
-                                                    const int *__restrict__ blk0,
-                                                    const int *__restrict__ rmap, int nrep,
-                                                    int nblk, int per_xcd, int ntot, StepArgs a)
+__global__ __launch_bounds__(BLOCK) void k_ens_step(
+    const RepGeo *__restrict__ reps, const int *__restrict__ p0,
+    const WorkGroup *__restrict__ wg, int nblk, int per_xcd, int ntot, StepArgs a)
 {
-    __shared__ unsigned hits[kHitCap * BLOCK];
+    __shared__ WaveLists lists[BLOCK / 64];
     const int it = xcd_cell(blockIdx.x, per_xcd);
     if (it >= nblk) return;
-    const int rl = replica_of(blk0, nrep, it);   // index in the launch's replica list
-    const int r = rmap[rl];
-    const int s = p0[r] + (it - blk0[rl]) * BLOCK + (int)threadIdx.x;
-    if (s >= p0[r + 1]) return;
+    const int r = wg[it].r;
+    int s = wg[it].s0 + (int)threadIdx.x;
+    const int end = p0[r + 1];
+    if (__builtin_amdgcn_readfirstlane(s) >= end) return;   // whole waves
+    const bool valid = s < end;
+    s = valid ? s : end - 1;
     // references into the replica table: local copies passed on by
     // reference would live in scratch memory
     const Geo &g = reps[r].g;
     const Pot &p = reps[r].p;
     const double radius = reps[r].radius;
     const int N = ntot;
-    const double xi = a.pos[s], yi = a.pos[N + s], zi = a.pos[2 * N + s];
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    SoAPos src{a.pos, N, radius};
-    StartTab tab{a.cstart};
-    Orig orig{a.id, 1, 0};
-    if (g.exact_mi)
-        gather_force<MASK, true, BLOCK>(g, p, src, tab, s, xi, yi, zi, radius,
-                                        hits + threadIdx.x, fx, fy, fz, a.err, orig);
-    else
-        gather_force<MASK, false, BLOCK>(g, p, src, tab, s, xi, yi, zi, radius,
-                                         hits + threadIdx.x, fx, fy, fz, a.err, orig);
+    wave_gather<MASK, 1>(g, p, reps[r].q, SoAPos{a.pos, N, radius}, StartTab{a.cstart}, a.upos, valid, s,
+                         lists[threadIdx.x >> 6], fx, fy, fz, a.err, Orig{a.id, 1, 0}, 0);
+    if (!valid) return;
     a.nfrc[s] = fx;
     a.nfrc[N + s] = fy;
     a.nfrc[2 * N + s] = fz;
@@ -109,14 +122,14 @@ __global__ __launch_bounds__(BLOCK) void k_ens_step(const RepGeo *__restrict__ r
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_ens_integ(const RepGeo *__restrict__ reps,
                                                      const int *__restrict__ p0,
-                                                     const int *__restrict__ blk0, int nrep,
+                                                     const WorkGroup *__restrict__ wg,
                                                      int nblk, int per_xcd, int ntot, GB gb,
                                                      StepArgs a)
 {
     const int it = xcd_cell(blockIdx.x, per_xcd);
     if (it >= nblk) return;
-    const int r = replica_of(blk0, nrep, it);
-    const int s = p0[r] + (it - blk0[r]) * BLOCK + (int)threadIdx.x;
+    const int r = wg[it].r;
+    const int s = wg[it].s0 + (int)threadIdx.x;
     if (s >= p0[r + 1]) return;
     const int N = ntot;
     integrate_one<false>(reps[r].g, gb, a, s, a.nfrc[s], a.nfrc[N + s], a.nfrc[2 * N + s]);
@@ -160,35 +173,31 @@ __global__ __launch_bounds__(kBrickThreads) void k_ens_step_brick(
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_ens_stats(const RepGeo *__restrict__ reps,
                                                      const int *__restrict__ p0,
-                                                     const int *__restrict__ blk0,
-                                                     const int *__restrict__ rmap, int nrep,
+                                                     const WorkGroup *__restrict__ wg,
                                                      int nblk, int per_xcd, int ntot,
-                                                     const double *pos, const int *id,
-                                                     const int *cstart, NbrStatsOut so)
+                                                     const double *pos, const uint4 *upos,
+                                                     const int *id, const int *cstart,
+                                                     NbrStatsOut so)
 {
-    __shared__ unsigned hits[kHitCap * BLOCK];
+    __shared__ WaveLists lists[BLOCK / 64];
     const int it = xcd_cell(blockIdx.x, per_xcd);
     if (it >= nblk) return;
-    const int rl = replica_of(blk0, nrep, it);
-    const int r = rmap[rl];
-    const int s = p0[r] + (it - blk0[rl]) * BLOCK + (int)threadIdx.x;
-    if (s >= p0[r + 1]) return;
+    const int r = wg[it].r;
+    int s = wg[it].s0 + (int)threadIdx.x;
+    const int end = p0[r + 1];
+    if (__builtin_amdgcn_readfirstlane(s) >= end) return;   // whole waves
+    const bool valid = s < end;
+    s = valid ? s : end - 1;
     const Geo &g = reps[r].g;
     const Pot &p = reps[r].p;
     const double radius = reps[r].radius;
     const int N = ntot;
-    const double xi = pos[s], yi = pos[N + s], zi = pos[2 * N + s];
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    SoAPos src{pos, N, radius};
-    StartTab tab{cstart};
-    Orig orig{id, 1, 0};
     NbrStats st;
-    if (g.exact_mi)
-        gather_force<F_CAL, true, BLOCK>(g, p, src, tab, s, xi, yi, zi, radius,
-                                         hits + threadIdx.x, fx, fy, fz, nullptr, orig, 0, &st);
-    else
-        gather_force<F_CAL, false, BLOCK>(g, p, src, tab, s, xi, yi, zi, radius,
-                                          hits + threadIdx.x, fx, fy, fz, nullptr, orig, 0, &st);
+    wave_gather<F_CAL, 1>(g, p, reps[r].q, SoAPos{pos, N, radius}, StartTab{cstart}, upos, valid, s,
+                          lists[threadIdx.x >> 6], fx, fy, fz, nullptr,
+                          Orig{id, 1, 0}, 0, &st);
+    if (!valid) return;
     so.count[id[s]] = st.count;
     so.hash[id[s]] = st.hash;
 }
@@ -276,7 +285,8 @@ struct EnsClass {
     int block = 256;           // thread-per-particle workgroup size
     int target = 192;          // brick kernel: home particles per brick
     int nblk = 0, nitems = 0;  // workgroups / bricks over the class's replicas
-    int *blk0 = nullptr, *item0 = nullptr;   // their prefixes over the list
+    WorkGroup *wg = nullptr;   // the workgroups (room for the smallest size)
+    int *item0 = nullptr;      // prefix of the replicas' brick counts
 };
 
 }  // namespace
@@ -294,7 +304,7 @@ struct psim_ens {
     EnsClass cls[kEnsClasses + 1];
     bool merged = false;
     int integ_nblk = 0;        // integrator: 256-lane workgroups over all replicas
-    int *integ_blk0 = nullptr; // prefix of the replicas' workgroup counts
+    WorkGroup *integ_wg = nullptr;
     std::vector<RepGeo> h_reps;
     std::vector<int> h_occ_n;
     hipStream_t stream = nullptr;
@@ -305,6 +315,8 @@ struct psim_ens {
     double *pos = nullptr, *pos0 = nullptr, *frc = nullptr, *mem = nullptr;
     double *npos = nullptr, *npos0 = nullptr, *nfrc = nullptr, *nmem = nullptr;
     double *vel = nullptr;
+    uint4 *upos = nullptr;       // box fractions and cells of pos
+    int *rep_of = nullptr;       // replica of slots 0, 256, 512, ...
     int *id = nullptr, *nid = nullptr, *key = nullptr, *arank = nullptr, *perm = nullptr;
     int *count = nullptr, *cstart = nullptr, *bsum = nullptr;
     // pos0 / frc / mem stay in the slot order of the last step (pos0: the
@@ -354,7 +366,7 @@ StepArgs ens_args(psim_ens *e)
 {
     StepArgs a{};
     a.pos = e->pos; a.pos0 = e->pos0; a.frc = e->frc; a.mem = e->mem;
-    a.id = e->id; a.cstart = e->cstart;
+    a.upos = e->upos; a.id = e->id; a.cstart = e->cstart;
     a.prev = e->lagged ? e->prev : nullptr;
     a.x0_raw = e->lagged ? 1 : 0;
     a.npos = e->npos; a.npos0 = e->npos0; a.nfrc = e->nfrc; a.nmem = e->nmem;
@@ -371,7 +383,7 @@ void launch_ens_pair(psim_ens *e, const EnsClass &cl, const StepArgs &a)
 {
     const int per = (cl.nblk + 7) / 8;
     k_ens_step<MASK, BLOCK><<<8 * per, BLOCK, 0, e->stream>>>(
-        e->reps, e->p0, cl.blk0, cl.rmap, (int)cl.reps.size(), cl.nblk, per, e->ntot, a);
+        e->reps, e->p0, cl.wg, cl.nblk, per, e->ntot, a);
 }
 
 // pair forces of one occupancy class's replicas into nfrc
@@ -401,8 +413,8 @@ void launch_ens_pair_block(psim_ens *e, const StepArgs &a)
     else
         for (int c = 0; c < kEnsClasses; ++c) launch_ens_pair_class<MASK>(e, e->cls[c], a);
     const int per = (e->integ_nblk + 7) / 8;
-    k_ens_integ<256><<<8 * per, 256, 0, e->stream>>>(e->reps, e->p0, e->integ_blk0, e->nrep,
-                                                     e->integ_nblk, per, e->ntot, e->gb, a);
+    k_ens_integ<256><<<8 * per, 256, 0, e->stream>>>(e->reps, e->p0, e->integ_wg, e->integ_nblk,
+                                                     per, e->ntot, e->gb, a);
 }
 
 // the buffer roles after one step's cell rebuild
@@ -435,12 +447,15 @@ void launch_build_ens(psim_ens *e, StepCtl *advance)
     // integrator, not after it); the positions this step started from become
     // pos0, and they, the forces and the memory stay where this step had or
     // wrote them: the next step reads them through prev
+    const ReplicaBox box{e->rep_of, e->p0, e->reps};
     if (n >= kMoveIlpMin)
         k_move_lagged<kMoveIlp><<<eblocks(n, 256 * kMoveIlp), 256, 0, st>>>(
-            n, e->perm, e->key, e->cstart, e->npos, e->id, e->pos0, e->nid, e->prev, advance);
+            n, e->perm, e->key, e->cstart, e->npos, e->id, e->pos0, e->nid, e->prev, advance,
+            e->upos, box);
     else
         k_move_lagged<1><<<eblocks(n, 256), 256, 0, st>>>(
-            n, e->perm, e->key, e->cstart, e->npos, e->id, e->pos0, e->nid, e->prev, advance);
+            n, e->perm, e->key, e->cstart, e->npos, e->id, e->pos0, e->nid, e->prev, advance,
+            e->upos, box);
     swap_lagged(e);
     e->lagged = true;
 }
@@ -463,40 +478,25 @@ int settle_ens(psim_ens *e)
     return 0;
 }
 
-// Workgroups of `block` lanes per replica for the thread-per-particle
-// kernel, and their prefix.
+// Workgroups of `block` lanes over the replicas `reps`.
+std::vector<WorkGroup> workgroups(const psim_ens *e, const std::vector<int> &reps, int block)
+{
+    std::vector<WorkGroup> wg;
+    for (int r : reps)
+        for (int s = e->h_p0[r]; s < e->h_p0[r + 1]; s += block) wg.push_back(WorkGroup{r, s});
+    return wg;
+}
+
 // Thread-per-particle workgroups of `block` lanes for the replicas of class c.
 int set_blocks(psim_ens *e, int c, int block)
 {
     EnsClass &cl = e->cls[c];
-    const int m = (int)cl.reps.size();
-    std::vector<int> b0(m + 1);
-    int nb = 0;
-    for (int l = 0; l < m; ++l) {
-        b0[l] = nb;
-        nb += (e->h_occ_n[cl.reps[l]] + block - 1) / block;
-    }
-    b0[m] = nb;
-    if (m) ECK(hipMemcpy(cl.blk0, b0.data(), sizeof(int) * (m + 1), hipMemcpyHostToDevice));
+    const std::vector<WorkGroup> wg = workgroups(e, cl.reps, block);
+    if (!wg.empty())
+        ECK(hipMemcpy(cl.wg, wg.data(), sizeof(WorkGroup) * wg.size(), hipMemcpyHostToDevice));
     cl.brick = false;
     cl.block = block;
-    cl.nblk = nb;
-    return 0;
-}
-
-// The integrator's 256-lane workgroups over all replicas.
-int set_integ_blocks(psim_ens *e)
-{
-    std::vector<int> b0(e->nrep + 1);
-    int nb = 0;
-    for (int r = 0; r < e->nrep; ++r) {
-        b0[r] = nb;
-        nb += (e->h_occ_n[r] + 255) / 256;
-    }
-    b0[e->nrep] = nb;
-    ECK(hipMemcpy(e->integ_blk0, b0.data(), sizeof(int) * (e->nrep + 1),
-                  hipMemcpyHostToDevice));
-    e->integ_nblk = nb;
+    cl.nblk = (int)wg.size();
     return 0;
 }
 
@@ -661,6 +661,7 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
         g.c0 = (int)ncell;
         h[r].g = g;
         h[r].p = p;
+        h[r].q = make_cull(g, p);
         h[r].radius = C.radius;
         h[r].bg = BrickGeo{};
         e->h_p0[r] = (int)ntot;
@@ -689,6 +690,16 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
     int **ibufs[] = {&e->id, &e->nid, &e->key, &e->arank, &e->perm, &e->prev};
     for (int **b : ibufs)
         if (!rc) rc = ealloc(b, (size_t)e->ntot);
+    if (!rc) rc = ealloc(&e->upos, (size_t)e->ntot);
+    std::vector<int> rep_of;
+    for (int t = 0, r = 0; t < e->ntot; t += 256) {
+        while (e->h_p0[r + 1] <= t) ++r;
+        rep_of.push_back(r);
+    }
+    if (!rc) rc = ealloc(&e->rep_of, rep_of.size());
+    if (!rc && hipMemcpy(e->rep_of, rep_of.data(), sizeof(int) * rep_of.size(),
+                         hipMemcpyHostToDevice) != hipSuccess)
+        rc = PSIM_E_HIP;
     if (!rc) rc = ealloc(&e->count, (size_t)e->ncell);
     if (!rc) rc = ealloc(&e->cstart, (size_t)e->ncell + 1);
     if (!rc) rc = ealloc(&e->bsum, (size_t)e->nscan);
@@ -696,7 +707,6 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
     if (!rc) rc = ealloc(&e->ctl, 1);
     if (!rc) rc = ealloc(&e->reps, (size_t)nrep);
     if (!rc) rc = ealloc(&e->p0, (size_t)nrep + 1);
-    if (!rc) rc = ealloc(&e->integ_blk0, (size_t)nrep + 1);
     e->h_reps = h;
     e->h_occ_n.resize(nrep);
     for (int r = 0; r < nrep; ++r) {
@@ -709,7 +719,7 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
         if (cl.reps.empty()) continue;
         const size_t m = cl.reps.size();
         rc = ealloc(&cl.rmap, m);
-        if (!rc) rc = ealloc(&cl.blk0, m + 1);
+        if (!rc) rc = ealloc(&cl.wg, workgroups(e, cl.reps, kEnsBlocks[0]).size());
         if (!rc) rc = ealloc(&cl.item0, m + 1);
         if (!rc && hipMemcpy(cl.rmap, cl.reps.data(), sizeof(int) * m, hipMemcpyHostToDevice) !=
                        hipSuccess)
@@ -718,7 +728,14 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
         if (!rc) rc = set_bricks(e, c, e->target);   // the replica table with its bricks
         if (!rc && !e->brick) rc = set_blocks(e, c, e->block);
     }
-    if (!rc) rc = set_integ_blocks(e);
+    if (!rc) {   // the integrator's workgroups: every replica, 256 lanes
+        const std::vector<WorkGroup> wg = workgroups(e, e->cls[kEnsClasses].reps, 256);
+        e->integ_nblk = (int)wg.size();
+        rc = ealloc(&e->integ_wg, wg.size());
+        if (!rc && hipMemcpy(e->integ_wg, wg.data(), sizeof(WorkGroup) * wg.size(),
+                             hipMemcpyHostToDevice) != hipSuccess)
+            rc = PSIM_E_HIP;
+    }
     if (!rc && hipMemcpy(e->p0, e->h_p0.data(), sizeof(int) * (nrep + 1), hipMemcpyHostToDevice) != hipSuccess)
         rc = PSIM_E_HIP;
     if (!rc && hipMemset(e->count, 0, sizeof(int) * e->ncell) != hipSuccess) rc = PSIM_E_HIP;
@@ -738,12 +755,12 @@ void psim_ens_destroy(psim_ens *e)
     drop_graph(e);
     void *bufs[] = {e->pos, e->pos0, e->frc, e->mem, e->npos, e->npos0, e->nfrc, e->nmem,
                     e->vel, e->id, e->nid, e->key, e->arank, e->perm, e->count, e->cstart,
-                    e->bsum, e->err, e->ctl, e->reps, e->p0, e->integ_blk0, e->st_count,
-                    e->st_hash, e->prev};
+                    e->bsum, e->err, e->ctl, e->reps, e->p0, e->integ_wg, e->st_count,
+                    e->st_hash, e->prev, e->upos, e->rep_of};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     for (EnsClass &cl : e->cls) {   // the occupancy classes and the all-replica one
-        void *cb[] = {cl.rmap, cl.blk0, cl.item0};
+        void *cb[] = {cl.rmap, cl.wg, cl.item0};
         for (void *b : cb)
             if (b) (void)hipFree(b);
     }
@@ -917,9 +934,8 @@ int psim_ens_pair_stats(psim_ens *e, int *count_by_orig, unsigned long long *has
         }
         const int per = (cl.nblk + 7) / 8;
 #define PSIM_ENS_STATS(BL)                                                                 \
-    k_ens_stats<BL><<<8 * per, BL, 0, e->stream>>>(e->reps, e->p0, cl.blk0, cl.rmap, m,    \
-                                                   cl.nblk, per, n, e->pos, e->id,         \
-                                                   e->cstart, so)
+    k_ens_stats<BL><<<8 * per, BL, 0, e->stream>>>(e->reps, e->p0, cl.wg, cl.nblk, per, n, \
+                                                   e->pos, e->upos, e->id, e->cstart, so)
         switch (cl.block) {
         case 64: PSIM_ENS_STATS(64); break;
         case 128: PSIM_ENS_STATS(128); break;

@@ -33,7 +33,10 @@ namespace {
 constexpr size_t kScratchBytes = PSIM_NOALLOC_SCRATCH_BYTES;
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) unsigned char scratch[kScratchBytes];
+// the working arrays of `carve`, then the box fractions of the sorted
+// positions (16 bytes for each of the particles that the former can hold)
+constexpr size_t kMaxParticles = kScratchBytes / 40;
+__device__ __align__(256) unsigned char scratch[kScratchBytes + 16 * kMaxParticles];
 
 // Device address of `scratch` on each GPU (each holds its own copy).
 std::mutex g_mu;
@@ -105,7 +108,8 @@ __global__ void k_hash_aos(Geo g, const double *pos3, int *key, int *rank, int *
 // gives an identity start); gathers the positions into slot order [3][N].
 __global__ void k_move_aos(int n, const int *__restrict__ perm, const int *__restrict__ key,
                            const int *__restrict__ cstart, const double *__restrict__ pos3,
-                           double *__restrict__ pos, int *__restrict__ id)
+                           double *__restrict__ pos, int *__restrict__ id,
+                           uint4 *__restrict__ upos, double inv_L)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
@@ -116,16 +120,18 @@ __global__ void k_move_aos(int n, const int *__restrict__ perm, const int *__res
     for (int u = b; u < e; ++u) rank += (perm[u] < s);
     const int dst = b + rank;
     const size_t q = 3 * (size_t)s;
-    pos[dst] = pos3[q];
-    pos[n + dst] = pos3[q + 1];
-    pos[2 * n + dst] = pos3[q + 2];
+    const double x = pos3[q], y = pos3[q + 1], z = pos3[q + 2];
+    pos[dst] = x;
+    pos[n + dst] = y;
+    pos[2 * n + dst] = z;
     id[dst] = s;
+    if (upos) upos[dst] = pack_position(x, y, z, c, inv_L);
 }
 
 template <int MASK>
-void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot,
-                       const PathChoice &path, const double *pos, const int *id,
-                       const int *cstart, double *fout, DevErr *err, hipStream_t st)
+void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot, const Cull &cull,
+                       const PathChoice &path, const double *pos, const uint4 *upos,
+                       const int *id, const int *cstart, double *fout, DevErr *err, hipStream_t st)
 {
     const int n = geo.n;
     if (path.dense) {
@@ -150,7 +156,7 @@ void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot,
             geo, pot, P.radius, path.bg, per, pos, id, cstart, fout, err);
     } else {
         k_forces<MASK, true><<<xcd_grid(eng::blocks_for(n, kBlock)), kBlock, 0, st>>>(
-            geo, pot, P.radius, pos, id, cstart, fout, err);
+            geo, pot, cull, P.radius, pos, upos, id, cstart, fout, err);
     }
 }
 
@@ -167,6 +173,7 @@ extern "C" int psim_gpu_forces_noalloc(const psim_params *params, const double *
     Pot pot;
     GB gb;
     make_constants(P, geo, pot, gb);
+    const Cull cull = make_cull(geo, pot);
     const int n = geo.n, ncell = geo.ncell;
     const int nscan = (ncell + kScanTile - 1) / kScanTile;
     const Carve cv = carve((size_t)n, (size_t)ncell, (size_t)nscan);
@@ -192,6 +199,8 @@ extern "C" int psim_gpu_forces_noalloc(const psim_params *params, const double *
     DevErr *err = reinterpret_cast<DevErr *>(b + cv.err);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const PathChoice path = choose_path(P, geo);
+    uint4 *upos = path.dense || path.brick ? nullptr
+                                           : reinterpret_cast<uint4 *>(b + kScratchBytes);
 
     // the previous call's contents: counts and the error record start at zero
     const int fill_blocks = (int)std::min<long long>(1024, eng::blocks_for(ncell, 256));
@@ -206,15 +215,16 @@ extern "C" int psim_gpu_forces_noalloc(const psim_params *params, const double *
     }
     k_scatter<1><<<eng::blocks_for(n, 256), 256, 0, st>>>(n, key, rank, cstart, perm,
                                                        direct ? count : nullptr, ncell);
-    k_move_aos<<<eng::blocks_for(n, 256), 256, 0, st>>>(n, perm, key, cstart, d_pos, pos, id);
+    k_move_aos<<<eng::blocks_for(n, 256), 256, 0, st>>>(n, perm, key, cstart, d_pos, pos, id,
+                                                         upos, cull.inv_L);
     switch (pot.mask) {
-    case 1: launch_forces_aos<1>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
-    case 2: launch_forces_aos<2>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
-    case 3: launch_forces_aos<3>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
-    case 4: launch_forces_aos<4>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
-    case 5: launch_forces_aos<5>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
-    case 6: launch_forces_aos<6>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
-    default: launch_forces_aos<7>(P, geo, pot, path, pos, id, cstart, d_force, err, st); break;
+    case 1: launch_forces_aos<1>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
+    case 2: launch_forces_aos<2>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
+    case 3: launch_forces_aos<3>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
+    case 4: launch_forces_aos<4>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
+    case 5: launch_forces_aos<5>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
+    case 6: launch_forces_aos<6>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
+    default: launch_forces_aos<7>(P, geo, pot, cull, path, pos, upos, id, cstart, d_force, err, st); break;
     }
     CK(hipGetLastError());
     DevErr h{};

@@ -71,6 +71,20 @@ inline GBCoeffs gb_coefficients(double kT, double gamma, double dt)
     return GBCoeffs{coeff0, coeff1, coeff2, coeff3, sig1, sig2, corr, dev, gn, goy2, goy3, hn};
 }
 
+// Each box fraction is truncated by less than one unit of 2^-32 box (r off by
+// less than sqrt(3) units) and the conversions and r^2 in FP32 add less than
+// 4e-7 relative; the bound is widened by four units of r and by 4e-6.
+inline Cull make_cull(const Geo &g, const Pot &p)
+{
+    Cull q;
+    q.inv_L = 1.0 / g.L;
+    q.inv_S2 = 1.0 / ((double)g.S * g.S);
+    q.inv_S = 1.0f / (float)g.S;
+    const double rc = std::sqrt(p.rc2_hi) * (4294967296.0 / g.L) + 4.0;
+    q.ucut2 = (float)(rc * rc * (1.0 + 4e-6));
+    return q;
+}
+
 inline void make_constants(const psim_params &P, Geo &g, Pot &p, GB &b)
 {
     g.n = P.n_particles;

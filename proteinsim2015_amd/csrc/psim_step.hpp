@@ -4,6 +4,7 @@
 
 #include "psim_brick.hpp"
 #include "psim_dense.hpp"
+#include "psim_gather.hpp"
 #include "psim_gpu.h"
 #include "psim_pairs.hpp"
 
@@ -70,6 +71,7 @@ inline PathChoice choose_path(const psim_params &P, const Geo &g)
 
 struct StepArgs {
     const double *pos, *pos0, *frc, *mem;
+    const uint4 *upos;   // box fractions and cells of pos (thread-per-particle kernels)
     const int *id, *cstart;
     const int *prev;     // slot of each particle in pos0 / frc / mem (null: the same slot)
     int x0_raw;          // pos0 holds the positions the last step started from (re-imaged
@@ -202,30 +204,24 @@ __device__ __forceinline__ void integrate_one(const Geo &g, const GB &gb, const 
 // where one lane per particle leaves most SIMDs idle and each lane waits
 // on 27 dependent cell lookups).
 template <int MASK, int BLOCK, int SPLIT = 1>
-__global__ __launch_bounds__(BLOCK) void k_step(Geo g, Pot p, GB gb, double radius,
-                                                StepArgs a)
+__global__ __launch_bounds__(BLOCK) void k_step(Geo g, Pot p, Cull q, GB gb,
+                                                double radius, StepArgs a)
 {
     static_assert(SPLIT >= 1 && 64 % SPLIT == 0 && (SPLIT & (SPLIT - 1)) == 0, "lane groups");
-    __shared__ unsigned hits[kHitCap * BLOCK];
+    __shared__ WaveLists lists[BLOCK / 64];
     const int t = xcd_block() * BLOCK + threadIdx.x;
-    const int s = t / SPLIT, sub = t % SPLIT;
-    if (s >= g.n) return;   // whole lane groups
+    const int sub = t % SPLIT;
+    int s = t / SPLIT;
+    if (__builtin_amdgcn_readfirstlane(s) >= g.n) return;   // whole waves
+    const bool valid = s < g.n;
+    s = valid ? s : g.n - 1;
     const int N = g.n;
-    const double xi = a.pos[s], yi = a.pos[N + s], zi = a.pos[2 * N + s];
     // the integrator's index loads, in flight during the force loop
     const int o = a.id[s], ps = a.prev ? a.prev[s] : s;
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    SoAPos src{a.pos, N, radius};
-    StartTab tab{a.cstart};
-    Orig orig{a.id, 1, 0};
-    if (g.exact_mi)
-        gather_force<MASK, true, BLOCK, SPLIT>(g, p, src, tab, s, xi, yi, zi, radius,
-                                               hits + threadIdx.x, fx, fy, fz, a.err, orig,
-                                               sub);
-    else
-        gather_force<MASK, false, BLOCK, SPLIT>(g, p, src, tab, s, xi, yi, zi, radius,
-                                                hits + threadIdx.x, fx, fy, fz, a.err, orig,
-                                                sub);
+    wave_gather<MASK, SPLIT>(g, p, q, SoAPos{a.pos, N, radius}, StartTab{a.cstart}, a.upos, valid,
+                             s, lists[threadIdx.x >> 6], fx, fy, fz, a.err, Orig{a.id, 1, 0},
+                             sub);
     // (not with LJ: its pair arithmetic leaves no registers for the pairs)
     if constexpr (SPLIT >= 4 && !(MASK & F_LJ)) {
         fx = split_sum<SPLIT>(fx);
@@ -240,21 +236,20 @@ __global__ __launch_bounds__(BLOCK) void k_step(Geo g, Pot p, GB gb, double radi
             const int base = (int)(threadIdx.x & 63u) & ~(SPLIT - 1);
             double z[6];
 #pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                z[2 * q] = __shfl(za, base + q, 64);
-                z[2 * q + 1] = __shfl(zb, base + q, 64);
+            for (int k = 0; k < 3; ++k) {
+                z[2 * k] = __shfl(za, base + k, 64);
+                z[2 * k + 1] = __shfl(zb, base + k, 64);
             }
-            if (sub != 0) return;
+            if (sub != 0 || !valid) return;
             integrate_one<true>(g, gb, a, s, fx, fy, fz, o, ps, z);
             return;
         }
-        if (sub != 0) return;
     } else if constexpr (SPLIT > 1) {
         fx = split_sum<SPLIT>(fx);
         fy = split_sum<SPLIT>(fy);
         fz = split_sum<SPLIT>(fz);
-        if (sub != 0) return;
     }
+    if (sub != 0 || !valid) return;
     integrate_one<true>(g, gb, a, s, fx, fy, fz, o, ps);
 }
 
@@ -329,27 +324,21 @@ __device__ __forceinline__ void store_force(double *fout, int N, int o, double f
 
 // Forces only at the current state, written by original index.
 template <int MASK, bool AOS = false>
-__global__ __launch_bounds__(kBlock) void k_forces(Geo g, Pot p, double radius,
-                                                   const double *pos, const int *id,
-                                                   const int *cstart, double *fout,
-                                                   DevErr *err)
+__global__ __launch_bounds__(kBlock) void k_forces(Geo g, Pot p, Cull q, double radius,
+                                                   const double *pos, const uint4 *upos,
+                                                   const int *id, const int *cstart,
+                                                   double *fout, DevErr *err)
 {
-    __shared__ unsigned hits[kHitCap * kBlock];
-    const int s = xcd_block() * kBlock + threadIdx.x;
-    if (s >= g.n) return;
+    __shared__ WaveLists lists[kBlock / 64];
+    int s = xcd_block() * kBlock + threadIdx.x;
+    if (__builtin_amdgcn_readfirstlane(s) >= g.n) return;   // whole waves
+    const bool valid = s < g.n;
+    s = valid ? s : g.n - 1;
     const int N = g.n;
-    const double xi = pos[s], yi = pos[N + s], zi = pos[2 * N + s];
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    SoAPos src{pos, N, radius};
-    StartTab tab{cstart};
-    Orig orig{id, 1, 0};
-    if (g.exact_mi)
-        gather_force<MASK, true>(g, p, src, tab, s, xi, yi, zi, radius,
-                                 hits + threadIdx.x, fx, fy, fz, err, orig);
-    else
-        gather_force<MASK, false>(g, p, src, tab, s, xi, yi, zi, radius,
-                                  hits + threadIdx.x, fx, fy, fz, err, orig);
-    store_force<AOS>(fout, N, id[s], fx, fy, fz);
+    wave_gather<MASK, 1>(g, p, q, SoAPos{pos, N, radius}, StartTab{cstart}, upos, valid, s,
+                         lists[threadIdx.x >> 6], fx, fy, fz, err, Orig{id, 1, 0}, 0);
+    if (valid) store_force<AOS>(fout, N, id[s], fx, fy, fz);
 }
 
 // Forces only, brick per workgroup (same result as k_forces).
@@ -398,31 +387,26 @@ __attribute__((amdgpu_waves_per_eu(dense_waves(MASK, LJN)))) void k_forces_dense
 // NbrStats instead of evaluated; counts and partner hashes by original index.
 // ---------------------------------------------------------------------------
 template <int BLOCK, int SPLIT>
-__global__ __launch_bounds__(BLOCK) void k_stats(Geo g, Pot p, double radius, const double *pos,
+__global__ __launch_bounds__(BLOCK) void k_stats(Geo g, Pot p, Cull q, double radius,
+                                                 const double *pos, const uint4 *upos,
                                                  const int *id, const int *cstart,
                                                  NbrStatsOut so)
 {
-    __shared__ unsigned hits[kHitCap * BLOCK];
+    __shared__ WaveLists lists[BLOCK / 64];
     const int t = xcd_block() * BLOCK + threadIdx.x;
-    const int s = t / SPLIT, sub = t % SPLIT;
-    if (s >= g.n) return;   // whole lane groups
+    const int sub = t % SPLIT;
+    int s = t / SPLIT;
+    if (__builtin_amdgcn_readfirstlane(s) >= g.n) return;   // whole waves
+    const bool valid = s < g.n;
+    s = valid ? s : g.n - 1;
     const int N = g.n;
-    const double xi = pos[s], yi = pos[N + s], zi = pos[2 * N + s];
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    SoAPos src{pos, N, radius};
-    StartTab tab{cstart};
-    Orig orig{id, 1, 0};
     NbrStats st;
-    if (g.exact_mi)
-        gather_force<F_CAL, true, BLOCK, SPLIT>(g, p, src, tab, s, xi, yi, zi, radius,
-                                                hits + threadIdx.x, fx, fy, fz, nullptr, orig,
-                                                sub, &st);
-    else
-        gather_force<F_CAL, false, BLOCK, SPLIT>(g, p, src, tab, s, xi, yi, zi, radius,
-                                                 hits + threadIdx.x, fx, fy, fz, nullptr, orig,
-                                                 sub, &st);
+    wave_gather<F_CAL, SPLIT>(g, p, q, SoAPos{pos, N, radius}, StartTab{cstart}, upos, valid, s,
+                              lists[threadIdx.x >> 6], fx, fy, fz, nullptr, Orig{id, 1, 0}, sub,
+                              &st);
     split_stats<SPLIT>(st);
-    if (sub == 0) {
+    if (sub == 0 && valid) {
         so.count[id[s]] = st.count;
         so.hash[id[s]] = st.hash;
     }
@@ -458,29 +442,42 @@ __global__ __launch_bounds__(kBrickThreads) void k_stats_brick(Geo g, Pot p, dou
                                                 sh, epi, &so);
 }
 
+// The cull's copy of the reference's sortedParticles.
+__global__ void k_pack_table(Geo g, double inv_L, const double *sorted4, uint4 *upos)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= g.n) return;
+    const AoS4Pos src{sorted4};
+    const double x = src.x(s), y = src.y(s), z = src.z(s);
+    upos[s] = pack_position(x, y, z,
+                            cell_1d(x, g.cell, g.S) + g.S * cell_1d(y, g.cell, g.S)
+                                + g.S2 * cell_1d(z, g.cell, g.S), inv_L);
+}
+
 // Forces from the reference's host arrays (IForce::getAcceleration over the
 // whole system): sorted4, particleHashIndex (hash, orig), cellStartEnd.
-template <int MASK>
-__global__ __launch_bounds__(kBlock) void k_forces_table(Geo g, Pot p,
-                                                         const double *sorted4,
-                                                         const int *hash_index,
-                                                         const int *cse, double *fout,
-                                                         DevErr *err)
+template <int MASK, int BLOCK, int SPLIT>
+__global__ __launch_bounds__(BLOCK) void k_forces_table(Geo g, Pot p, Cull q, const double *sorted4,
+                                                        const uint4 *upos,
+                                                        const int *hash_index, const int *cse,
+                                                        double *fout, DevErr *err)
 {
-    __shared__ unsigned hits[kHitCap * kBlock];
-    const int s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= g.n) return;
-    AoS4Pos src{sorted4};
-    PairTab tab{cse};
-    Orig orig{hash_index, 2, 1};
-    const double xi = src.x(s), yi = src.y(s), zi = src.z(s), ri = src.rad(s);
+    __shared__ WaveLists lists[BLOCK / 64];
+    const int t = xcd_block() * BLOCK + threadIdx.x;
+    const int sub = t % SPLIT;
+    int s = t / SPLIT;
+    if (__builtin_amdgcn_readfirstlane(s) >= g.n) return;   // whole waves
+    const bool valid = s < g.n;
+    s = valid ? s : g.n - 1;
+    const AoS4Pos src{sorted4};
+    const Orig orig{hash_index, 2, 1};
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    if (g.exact_mi)
-        gather_force<MASK, true>(g, p, src, tab, s, xi, yi, zi, ri,
-                                 hits + threadIdx.x, fx, fy, fz, err, orig);
-    else
-        gather_force<MASK, false>(g, p, src, tab, s, xi, yi, zi, ri,
-                                  hits + threadIdx.x, fx, fy, fz, err, orig);
+    wave_gather<MASK, SPLIT>(g, p, q, src, PairTab{cse}, upos, valid, s, lists[threadIdx.x >> 6],
+                             fx, fy, fz, err, orig, sub);
+    fx = split_sum<SPLIT>(fx);
+    fy = split_sum<SPLIT>(fy);
+    fz = split_sum<SPLIT>(fz);
+    if (sub != 0 || !valid) return;
     const int o = orig(s);
     fout[3 * (size_t)o] = fx;   // particleForce[3*orig + k] (LJPotential.cpp:179-181)
     fout[3 * (size_t)o + 1] = fy;
