@@ -248,11 +248,21 @@ void launch_forces_mask(psim_ctx *c)
         });
     } else if (c->brick) {
         const int per = (c->bg.nbricks + 7) / 8;
-        k_forces_brick<MASK><<<8 * per, kBrickThreads, 0, c->stream>>>(
-            c->geo, c->pot, c->prm.radius, c->bg, per, c->pos, c->id, c->cstart, c->fout,
-            c->err);
+        if (c->brick_g == 1)
+            k_forces_brick<MASK, 1><<<8 * per, kBrickThreads, 0, c->stream>>>(
+                c->geo, c->pot, c->prm.radius, c->bg, per, c->pos, c->id, c->cstart, c->fout,
+                c->err);
+        else
+            k_forces_brick<MASK, kSmallSplit><<<8 * per, kBrickThreads, 0, c->stream>>>(
+                c->geo, c->pot, c->prm.radius, c->bg, per, c->pos, c->id, c->cstart, c->fout,
+                c->err);
+    } else if (c->n < kSmallSystem) {
+        k_forces<MASK, 64, kSmallSplit>
+            <<<xcd_grid(blocks_for((long long)c->n * kSmallSplit, 64)), 64, 0, c->stream>>>(
+                c->geo, c->pot, c->cull, c->prm.radius, c->pos, c->upos, c->id, c->cstart,
+                c->fout, c->err);
     } else {
-        k_forces<MASK><<<xcd_grid(blocks_for(c->n, kBlock)), kBlock, 0, c->stream>>>(
+        k_forces<MASK, kBlock, 1><<<xcd_grid(blocks_for(c->n, kBlock)), kBlock, 0, c->stream>>>(
             c->geo, c->pot, c->cull, c->prm.radius, c->pos, c->upos, c->id, c->cstart, c->fout,
             c->err);
     }

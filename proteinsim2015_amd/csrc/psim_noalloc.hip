@@ -152,11 +152,20 @@ void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot, con
         launch(std::integral_constant<int, 0>{});
     } else if (path.brick) {
         const int per = (path.bg.nbricks + 7) / 8;
-        k_forces_brick<MASK, true><<<8 * per, kBrickThreads, 0, st>>>(
-            geo, pot, P.radius, path.bg, per, pos, id, cstart, fout, err);
+        if (path.brick_g == 1)
+            k_forces_brick<MASK, 1, true><<<8 * per, kBrickThreads, 0, st>>>(
+                geo, pot, P.radius, path.bg, per, pos, id, cstart, fout, err);
+        else
+            k_forces_brick<MASK, kSmallSplit, true><<<8 * per, kBrickThreads, 0, st>>>(
+                geo, pot, P.radius, path.bg, per, pos, id, cstart, fout, err);
+    } else if (n < kSmallSystem) {
+        k_forces<MASK, 64, kSmallSplit, true>
+            <<<xcd_grid(eng::blocks_for((long long)n * kSmallSplit, 64)), 64, 0, st>>>(
+                geo, pot, cull, P.radius, pos, upos, id, cstart, fout, err);
     } else {
-        k_forces<MASK, true><<<xcd_grid(eng::blocks_for(n, kBlock)), kBlock, 0, st>>>(
-            geo, pot, cull, P.radius, pos, upos, id, cstart, fout, err);
+        k_forces<MASK, kBlock, 1, true>
+            <<<xcd_grid(eng::blocks_for(n, kBlock)), kBlock, 0, st>>>(
+                geo, pot, cull, P.radius, pos, upos, id, cstart, fout, err);
     }
 }
 

@@ -2,6 +2,9 @@
 // kernel paths), the G&B integrator epilogue and force-only evaluations.
 #pragma once
 
+#include <algorithm>
+#include <cmath>
+
 #include "psim_brick.hpp"
 #include "psim_dense.hpp"
 #include "psim_gather.hpp"
@@ -11,8 +14,20 @@
 namespace psim {
 namespace {
 
-// mean particles per cell above which the cell-per-workgroup kernel is used
-constexpr double kDenseMinOccupancy = 2.0;
+// Mean particles per cell from which the cell-per-workgroup kernel beats the
+// thread-per-particle one.  The former's time grows with the cells (a
+// workgroup each, of which the chip holds 1792 at once), the latter's with the
+// candidates per particle, at four lanes per particle below kSmallSystem and
+// one above.  Measured on MI355X, whole steps (thread per particle / cell per
+// workgroup, us): N = 4096 at 2.4 per cell 21 / 24, at 3.1 26 / 24; 16,384 at
+// 4.0 33 / 35, at 4.9 36 / 31; 32,768 at 3.1 33 / 52, at 6.7 45 / 36; 65,536 at
+// 5.4 55 / 59, at 6.2 59 / 55; 262,144 at 6.1 117 / 151, at 8.0 149 / 143;
+// 1,048,576 at 3.1 249 / 1016, at 7.9 518 / 510, at 9.5 566 / 425.
+inline double dense_min_occupancy(int n)
+{
+    if (n >= 256 * 1024) return 8.0;
+    return std::min(5.7, std::max(2.7, 2.7 + std::log2(n / 6144.0)));
+}
 // below this many particles the thread-per-particle kernels use 64-lane
 // blocks (256-lane blocks would leave CUs idle: 256 CUs x 4 blocks)
 constexpr int kSmallSystem = 256 * 1024;
@@ -43,7 +58,7 @@ inline int check_params(const psim_params &P)
 
 // Pair-kernel path of a system: the cell-per-workgroup kernel needs S >= 4
 // (shifted image = minimum image) and pays off once cells hold a few
-// particles; below that, one thread per particle (bricks of cells per
+// particles (dense_min_occupancy); below that, one thread per particle (bricks of cells per
 // workgroup, path 3, give the same bits but measured slower at every sparse
 // density).
 struct PathChoice {
@@ -61,7 +76,7 @@ inline PathChoice choose_path(const psim_params &P, const Geo &g)
     else if (P.kernel_path == 2)
         c.dense = g.S >= 4;
     else
-        c.dense = g.S >= 4 && occupancy >= kDenseMinOccupancy;
+        c.dense = g.S >= 4 && occupancy >= dense_min_occupancy(g.n);
     c.brick = P.kernel_path == 3;
     c.brick_g = g.n < kSmallSystem ? kSmallSplit : 1;
     c.bg = brick_shape(g.S, occupancy, kBrickTarget * kBrickThreads / c.brick_g);
@@ -323,26 +338,31 @@ __device__ __forceinline__ void store_force(double *fout, int N, int o, double f
 }
 
 // Forces only at the current state, written by original index.
-template <int MASK, bool AOS = false>
-__global__ __launch_bounds__(kBlock) void k_forces(Geo g, Pot p, Cull q, double radius,
+template <int MASK, int BLOCK, int SPLIT, bool AOS = false>
+__global__ __launch_bounds__(BLOCK) void k_forces(Geo g, Pot p, Cull q, double radius,
                                                    const double *pos, const uint4 *upos,
                                                    const int *id, const int *cstart,
                                                    double *fout, DevErr *err)
 {
-    __shared__ WaveLists lists[kBlock / 64];
-    int s = xcd_block() * kBlock + threadIdx.x;
+    __shared__ WaveLists lists[BLOCK / 64];
+    const int t = xcd_block() * BLOCK + threadIdx.x;
+    const int sub = t % SPLIT;
+    int s = t / SPLIT;
     if (__builtin_amdgcn_readfirstlane(s) >= g.n) return;   // whole waves
     const bool valid = s < g.n;
     s = valid ? s : g.n - 1;
     const int N = g.n;
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    wave_gather<MASK, 1>(g, p, q, SoAPos{pos, N, radius}, StartTab{cstart}, upos, valid, s,
-                         lists[threadIdx.x >> 6], fx, fy, fz, err, Orig{id, 1, 0}, 0);
-    if (valid) store_force<AOS>(fout, N, id[s], fx, fy, fz);
+    wave_gather<MASK, SPLIT>(g, p, q, SoAPos{pos, N, radius}, StartTab{cstart}, upos, valid, s,
+                             lists[threadIdx.x >> 6], fx, fy, fz, err, Orig{id, 1, 0}, sub);
+    fx = split_sum<SPLIT>(fx);
+    fy = split_sum<SPLIT>(fy);
+    fz = split_sum<SPLIT>(fz);
+    if (sub == 0 && valid) store_force<AOS>(fout, N, id[s], fx, fy, fz);
 }
 
-// Forces only, brick per workgroup (same result as k_forces).
-template <int MASK, bool AOS = false>
+// Forces only, brick per workgroup (same result as k_forces with SPLIT = G).
+template <int MASK, int G, bool AOS = false>
 __global__ __launch_bounds__(kBrickThreads) void k_forces_brick(Geo g, Pot p, double radius,
                                                                 BrickGeo bg, int per_xcd,
                                                                 const double *pos,
@@ -358,9 +378,9 @@ __global__ __launch_bounds__(kBrickThreads) void k_forces_brick(Geo g, Pot p, do
         store_force<AOS>(fout, N, id[s], fx, fy, fz);
     };
     if (g.exact_mi)
-        brick_forces<MASK, true, 1>(g, p, radius, pos, cstart, id, err, bg, b, sh, epi);
+        brick_forces<MASK, true, G>(g, p, radius, pos, cstart, id, err, bg, b, sh, epi);
     else
-        brick_forces<MASK, false, 1>(g, p, radius, pos, cstart, id, err, bg, b, sh, epi);
+        brick_forces<MASK, false, G>(g, p, radius, pos, cstart, id, err, bg, b, sh, epi);
 }
 
 template <int MASK, int LJN, bool AOS = false>
