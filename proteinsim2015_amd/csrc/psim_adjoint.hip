@@ -342,11 +342,27 @@ __global__ void k_gather_slots(int n, const int *id, const double *in, double *o
     for (int d = 0; d < 3; ++d) out[(size_t)d * n + s] = in[(size_t)d * n + o];
 }
 
-// lam = alpha * a1 (the last step: a_{K+1} = 0)
-__global__ void k_scale(int n3, double alpha, const double *a, double *out)
+// The end of the trajectory: a1 = gx (n x 3 by original index) as [3][n],
+// a2 = 0, lam = alpha a1
+__global__ void k_adj_start(int n, double alpha, const double *gx, double *a1, double *a2,
+                            double *lam)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n3) out[i] = alpha * a[i];
+    const int o = blockIdx.x * blockDim.x + threadIdx.x;
+    if (o >= n) return;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double v = gx[3 * (size_t)o + d];
+        a1[(size_t)d * n + o] = v;
+        a2[(size_t)d * n + o] = 0.0;
+        lam[(size_t)d * n + o] = alpha * v;
+    }
+}
+
+// [3][n] to n x 3
+__global__ void k_aos(int n, const double *v, double *out)
+{
+    const int o = blockIdx.x * blockDim.x + threadIdx.x;
+    if (o < n) store_aos(out, o, v[o], v[(size_t)n + o], v[2 * (size_t)n + o]);
 }
 
 }  // namespace
@@ -729,17 +745,12 @@ int psim_adj_backward(psim_adjoint *A, const double *gx, double *dtheta, double 
     const AdjPot q = make_adj(c->prm, A->win);
     // a_K = gx, a_{K+1} = 0, lambda_{K-1} = alpha_{K-1} a_K
     {
-        std::vector<double> h(n3);
-        for (int o = 0; o < n; ++o)
-            for (int d = 0; d < 3; ++d) h[(size_t)d * n + o] = gx[3 * (size_t)o + d];
-        CK(hipMemcpyAsync(A->a[1], h.data(), sizeof(double) * n3, hipMemcpyHostToDevice,
-                          c->stream));
-        CK(hipStreamSynchronize(c->stream));
+        const Xfer x{const_cast<double *>(gx), A->lam[1], sizeof(double) * n3};
+        if (stage_write(c->stage, c->stream, &x, 1)) return PSIM_E_HIP;
     }
-    CK(hipMemsetAsync(A->a[2], 0, sizeof(double) * n3, c->stream));
     const size_t nbk = adj_blocks(c);
-    k_scale<<<blocks_for((long long)n3, 256), 256, 0, c->stream>>>((int)n3, alpha(A->K - 1),
-                                                                   A->a[1], A->lam[0]);
+    k_adj_start<<<blocks_for(n, 256), 256, 0, c->stream>>>(n, alpha(A->K - 1), A->lam[1], A->a[1],
+                                                           A->a[2], A->lam[0]);
     CK(hipGetLastError());
     double *a0 = A->a[0], *a1 = A->a[1], *a2 = A->a[2];
     double *lam = A->lam[0], *lam_prev = A->lam[1];
@@ -810,17 +821,12 @@ int psim_adj_backward(psim_adjoint *A, const double *gx, double *dtheta, double 
     k_theta_sum<<<kNTheta, 256, 0, c->stream>>>(A->acc + kNTheta, kThetaChunks, A->acc);
     CK(hipGetLastError());
     // a1 now holds a_0 = dL/dx_0
-    std::vector<double> h(gx0 ? n3 : 0);
-    if (gx0)
-        CK(hipMemcpyAsync(h.data(), a1, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-    CK(hipMemcpyAsync(dtheta, A->acc, sizeof(double) * kNTheta, hipMemcpyDeviceToHost,
-                      c->stream));
+    if (gx0) k_aos<<<blocks_for(n, 256), 256, 0, c->stream>>>(n, a1, a0);
     // leave the context at the end of the trajectory
     if ((rc = restore_cp(A, A->ncp))) return rc;
-    CK(hipStreamSynchronize(c->stream));
-    if (gx0)
-        for (int o = 0; o < n; ++o)
-            for (int d = 0; d < 3; ++d) gx0[3 * (size_t)o + d] = h[(size_t)d * n + o];
+    const Xfer x[2] = {{dtheta, A->acc, sizeof(double) * kNTheta},
+                       {gx0, a0, sizeof(double) * n3}};
+    if (stage_read(c->stage, c->stream, x, gx0 ? 2 : 1)) return PSIM_E_HIP;
     return 0;
 }
 

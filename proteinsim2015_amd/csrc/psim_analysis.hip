@@ -359,10 +359,7 @@ __global__ __launch_bounds__(kAnaBlock) void k_pair_hist_grad(HistGeo h, const d
         gy += c * dy;
         gz += c * dz;
     });
-    const int o = id[s];
-    grad[o] = gx;
-    grad[N + o] = gy;
-    grad[2 * N + o] = gz;
+    store_aos(grad, id[s], gx, gy, gz);
 }
 
 // canonical within-cell order of the histogram grid (ascending slot), so the
@@ -565,10 +562,7 @@ __global__ __launch_bounds__(kAnaBlock) void k_pair_hist_grad_grid(
         gz += __shfl_xor(gz, d, 64);
     }
     if (sub == 0) {
-        const int o = id[perm[t]];
-        grad[o] = gx;
-        grad[N + o] = gy;
-        grad[2 * N + o] = gz;
+        store_aos(grad, id[perm[t]], gx, gy, gz);
     }
 }
 
@@ -781,12 +775,9 @@ int psim_gpu_observables(psim_ctx *c, double contact_r, psim_observables *out,
                                                    c->iwork, c->work);
     CK(hipGetLastError());
     std::vector<double> part((size_t)nb * 4);
-    CK(hipMemcpyAsync(part.data(), c->work, sizeof(double) * part.size(),
-                      hipMemcpyDeviceToHost, c->stream));
-    if (coord_by_orig)
-        CK(hipMemcpyAsync(coord_by_orig, c->iwork, sizeof(int) * n, hipMemcpyDeviceToHost,
-                          c->stream));
-    CK(hipStreamSynchronize(c->stream));
+    const Xfer x[2] = {{part.data(), c->work, sizeof(double) * part.size()},
+                       {coord_by_orig, c->iwork, sizeof(int) * (size_t)n}};
+    if (stage_read(c->stage, c->stream, x, coord_by_orig ? 2 : 1)) return PSIM_E_HIP;
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
     for (unsigned b = 0; b < nb; ++b)
         for (int q = 0; q < 4; ++q) sum[q] += part[(size_t)b * 4 + q];
@@ -819,13 +810,13 @@ int psim_gpu_clusters(psim_ctx *c, double contact_r, int min_size, int *labels_b
         k_cc_jump<<<blocks_for(n, 256), 256, 0, c->stream>>>(n, lab);
         CK(hipGetLastError());
         int hc = 0;
-        CK(hipMemcpyAsync(&hc, changed, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        CK(hipStreamSynchronize(c->stream));
+        const Xfer x{&hc, changed, sizeof(int)};
+        if (stage_read(c->stage, c->stream, &x, 1)) return PSIM_E_HIP;
         if (!hc) break;
     }
     std::vector<int> lh(n);
-    CK(hipMemcpyAsync(lh.data(), lab, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-    CK(hipStreamSynchronize(c->stream));
+    const Xfer x{lh.data(), lab, sizeof(int) * (size_t)n};
+    if (stage_read(c->stage, c->stream, &x, 1)) return PSIM_E_HIP;
     if (labels_by_orig) std::memcpy(labels_by_orig, lh.data(), sizeof(int) * n);
     // writeClusters (analysisCluster.cpp:86-100): clusters of more than
     // min_size - 1 members, average size by integer division
@@ -864,10 +855,8 @@ int psim_gpu_pair_histogram(psim_ctx *c, double r_lo, double width, int nbins, d
                                                                         c->hg.cstart, part);
         k_hist_sum<<<nbins, 256, 0, c->stream>>>(part, (int)nblk, nbins, out);
         CK(hipGetLastError());
-        CK(hipMemcpyAsync(hist, out, sizeof(double) * nbins, hipMemcpyDeviceToHost,
-                          c->stream));
-        CK(hipStreamSynchronize(c->stream));
-        return 0;
+        const Xfer x{hist, out, sizeof(double) * (size_t)nbins};
+        return stage_read(c->stage, c->stream, &x, 1) ? PSIM_E_HIP : 0;
     }
     rc = ensure_work(c, (size_t)nbins, 1);
     if (rc) return rc;
@@ -875,10 +864,8 @@ int psim_gpu_pair_histogram(psim_ctx *c, double r_lo, double width, int nbins, d
     k_pair_hist<<<blocks_for(n, kAnaBlock), kAnaBlock, 0, c->stream>>>(
         h, c->pos, c->hg.perm, c->hg.cstart, c->work);
     CK(hipGetLastError());
-    CK(hipMemcpyAsync(hist, c->work, sizeof(double) * nbins, hipMemcpyDeviceToHost,
-                      c->stream));
-    CK(hipStreamSynchronize(c->stream));
-    return 0;
+    const Xfer x{hist, c->work, sizeof(double) * (size_t)nbins};
+    return stage_read(c->stage, c->stream, &x, 1) ? PSIM_E_HIP : 0;
 }
 
 int psim_gpu_pair_histogram_grad(psim_ctx *c, double r_lo, double width, int nbins,
@@ -894,7 +881,8 @@ int psim_gpu_pair_histogram_grad(psim_ctx *c, double r_lo, double width, int nbi
     rc = ensure_work(c, (size_t)nbins + 3 * (size_t)n, 1);
     if (rc) return rc;
     double *dw = c->work, *dg = c->work + nbins;
-    CK(hipMemcpyAsync(dw, w, sizeof(double) * nbins, hipMemcpyHostToDevice, c->stream));
+    const Xfer xw{const_cast<double *>(w), dw, sizeof(double) * (size_t)nbins};
+    if (stage_write(c->stage, c->stream, &xw, 1)) return PSIM_E_HIP;
     if (h.S) {
         const size_t lds = sizeof(double) * (nbins + 1);
         k_pair_hist_grad_grid<kHistSplit>
@@ -905,13 +893,8 @@ int psim_gpu_pair_histogram_grad(psim_ctx *c, double r_lo, double width, int nbi
             h, c->pos, c->hg.perm, c->hg.cstart, c->id, dw, dg);
     }
     CK(hipGetLastError());
-    std::vector<double> hg(3 * (size_t)n);
-    CK(hipMemcpyAsync(hg.data(), dg, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
-                      c->stream));
-    CK(hipStreamSynchronize(c->stream));
-    for (int o = 0; o < n; ++o)
-        for (int d = 0; d < 3; ++d) grad[3 * (size_t)o + d] = hg[(size_t)d * n + o];
-    return 0;
+    const Xfer x{grad, dg, sizeof(double) * 3 * (size_t)n};
+    return stage_read(c->stage, c->stream, &x, 1) ? PSIM_E_HIP : 0;
 }
 
 }  // extern "C"

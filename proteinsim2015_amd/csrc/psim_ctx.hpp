@@ -10,6 +10,7 @@
 #include "psim_brick_shape.hpp"
 #include "psim_device.hpp"
 #include "psim_gpu.h"
+#include "psim_stage.hpp"
 
 // The buffers and constants a captured step sequence bakes into its kernels.
 struct GraphKey {
@@ -95,6 +96,7 @@ struct psim_ctx {
         int *id = nullptr, *cstart = nullptr;
         int *inv = nullptr;   // original index -> slot
     } rec;
+    psim::HostStage stage;      // pinned copies to and from the caller
     double *work = nullptr;     // analysis scratch (partials, histograms)
     size_t work_cap = 0;        // doubles
     int *iwork = nullptr;       // analysis scratch (labels, flags)

@@ -155,6 +155,35 @@ int settle(psim_ctx *c)
     return 0;
 }
 
+// The state as n x 3 arrays by original index, the previous positions, forces
+// and memory read where the last step left them (prev and raw pos0 as
+// integrate_one reads them).  Null outputs are skipped.
+__global__ void k_export_state(int n, const int *__restrict__ id, const int *__restrict__ prev,
+                               int x0_raw, double L, const double *__restrict__ pos,
+                               const double *__restrict__ pos0, const double *__restrict__ vel,
+                               const double *__restrict__ frc, const double *__restrict__ mem,
+                               double *pos_out, double *pos0_out, double *vel_out,
+                               double *frc_out, double *mem_out)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    const int o = id[s], p = prev ? prev[s] : s;
+    const double x = pos[s], y = pos[n + s], z = pos[2 * n + s];
+    if (pos_out) store_aos(pos_out, o, x, y, z);
+    if (pos0_out) {
+        double x0 = pos0[p], y0 = pos0[n + p], z0 = pos0[2 * n + p];
+        if (x0_raw) {
+            x0 = safe_mod0(x0, x, L);
+            y0 = safe_mod0(y0, y, L);
+            z0 = safe_mod0(z0, z, L);
+        }
+        store_aos(pos0_out, o, x0, y0, z0);
+    }
+    if (frc_out) store_aos(frc_out, o, frc[p], frc[n + p], frc[2 * n + p]);
+    if (mem_out) store_aos(mem_out, o, mem[p], mem[n + p], mem[2 * n + p]);
+    if (vel_out) store_aos(vel_out, s, vel[s], vel[n + s], vel[2 * n + s]);   // by original index
+}
+
 __global__ void k_pack(Geo g, double inv_L, const double *pos, uint4 *upos)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -488,12 +517,22 @@ int run_steps(psim_ctx *c, int nsteps, const double *d_noise)
 int read_error(psim_ctx *c, int *code, int *i, int *j)
 {
     DevErr h{};
-    CK(hipMemcpyAsync(&h, c->err, sizeof(DevErr), hipMemcpyDeviceToHost, c->stream));
-    CK(hipStreamSynchronize(c->stream));
+    const Xfer x{&h, c->err, sizeof(DevErr)};
+    if (stage_read(c->stage, c->stream, &x, 1)) return PSIM_E_HIP;
     if (code) *code = h.code;
     if (i) *i = h.i;
     if (j) *j = h.j;
     return 0;
+}
+
+// The forces a force kernel left in fout (n x 3) and the error record in one
+// copy; returns the error code.
+int read_forces(psim_ctx *c, double *force_out)
+{
+    DevErr h{};
+    const Xfer x[2] = {{force_out, c->fout, sizeof(double) * 3 * (size_t)c->n},
+                       {&h, c->err, sizeof(DevErr)}};
+    return stage_read(c->stage, c->stream, x, 2) ? PSIM_E_HIP : h.code;
 }
 
 }  // namespace
@@ -675,6 +714,8 @@ int psim_gpu_create(const psim_params *params, psim_ctx **out)
         rc = PSIM_E_HIP;
     if (!rc && hipMemsetAsync(c->err, 0, sizeof(DevErr), c->stream) != hipSuccess)
         rc = PSIM_E_HIP;
+    // the five arrays of a state, each at an aligned place
+    if (!rc && !stage_reserve(c->stage, 5 * (sizeof(double) * n3 + 64))) rc = PSIM_E_HIP;
     if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PSIM_E_HIP;
     if (rc) {
         psim_gpu_destroy(c);
@@ -728,6 +769,7 @@ void psim_gpu_destroy(psim_ctx *c)
                     c->work, c->iwork};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    stage_free(c->stage);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -750,30 +792,25 @@ int psim_gpu_get_state(psim_ctx *c, double *pos, double *pos0, double *vel, doub
                        int *vel_counter, unsigned long long *step_index)
 {
     if (!c || !c->have_state) return PSIM_E_ARG;
-    int rs = psim::eng::settle(c);
-    if (rs) return rs;
     const int n = c->n;
-    std::vector<int> ids(n);
-    std::vector<double> h(3 * (size_t)n);
-    CK(hipMemcpyAsync(ids.data(), c->id, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-    CK(hipStreamSynchronize(c->stream));
-    auto aos = [&](const double *src, double *dst, bool by_slot) -> int {
-        if (!dst) return 0;
-        CK(hipMemcpyAsync(h.data(), src, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
-                          c->stream));
-        CK(hipStreamSynchronize(c->stream));
-        for (int s = 0; s < n; ++s) {
-            int o = by_slot ? ids[s] : s;
-            for (int d = 0; d < 3; ++d) dst[3 * (size_t)o + d] = h[(size_t)d * n + s];
-        }
-        return 0;
-    };
-    int rc;
-    if ((rc = aos(c->pos, pos, true))) return rc;
-    if ((rc = aos(c->pos0, pos0, true))) return rc;
-    if ((rc = aos(c->vel, vel, false))) return rc;
-    if ((rc = aos(c->frc, frc, true))) return rc;
-    if ((rc = aos(c->mem, memx, true))) return rc;
+    // n x 3 arrays made on the device in buffers that hold nothing between
+    // steps, then copied out through pinned memory
+    double *dst[5] = {pos, pos0, vel, frc, memx};
+    double *out[5] = {c->npos, c->npos0, c->fout, c->nfrc, c->nmem};
+    const size_t b = sizeof(double) * 3 * (size_t)n;
+    Xfer x[5];
+    int nx = 0;
+    for (int k = 0; k < 5; ++k) {
+        if (dst[k])
+            x[nx++] = Xfer{dst[k], out[k], b};
+        else
+            out[k] = nullptr;
+    }
+    k_export_state<<<blocks_for(n, 256), 256, 0, c->stream>>>(
+        n, c->id, c->lagged ? c->prev : nullptr, c->lagged ? 1 : 0, c->prm.box, c->pos, c->pos0,
+        c->vel, c->frc, c->mem, out[0], out[1], out[2], out[3], out[4]);
+    CK(hipGetLastError());
+    if (stage_read(c->stage, c->stream, x, nx)) return PSIM_E_HIP;
     if (frc0) {
         // frc0 of the last integrator call is not retained on the device
         for (size_t k = 0; k < 3 * (size_t)n; ++k) frc0[k] = std::nan("");
@@ -799,8 +836,8 @@ int psim_gpu_step(psim_ctx *c, int nsteps, const double *noise)
             if (rc) return rc;
             c->noise_cap = need;
         }
-        CK(hipMemcpyAsync(c->noise, noise, need * sizeof(double), hipMemcpyHostToDevice,
-                          c->stream));
+        const Xfer x{const_cast<double *>(noise), c->noise, need * sizeof(double)};
+        if (stage_write(c->stage, c->stream, &x, 1)) return PSIM_E_HIP;
         d_noise = c->noise;
     }
     int rc = run_steps(c, nsteps, d_noise);
@@ -831,16 +868,7 @@ int psim_gpu_forces(psim_ctx *c, double *force_out)
     default: return PSIM_E_ARG;
     }
     CK(hipGetLastError());
-    const int n = c->n;
-    std::vector<double> h(3 * (size_t)n);
-    CK(hipMemcpyAsync(h.data(), c->fout, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
-                      c->stream));
-    CK(hipStreamSynchronize(c->stream));
-    for (int i = 0; i < n; ++i)
-        for (int d = 0; d < 3; ++d) force_out[3 * (size_t)i + d] = h[(size_t)d * n + i];
-    int code = 0;
-    int rc = read_error(c, &code, nullptr, nullptr);
-    return rc ? rc : code;
+    return read_forces(c, force_out);
 }
 
 int psim_gpu_force_table(psim_ctx *c, const double *sorted4, const int *hash_index,
@@ -850,15 +878,16 @@ int psim_gpu_force_table(psim_ctx *c, const double *sorted4, const int *hash_ind
     const int n = c->n;
     // the kernel indexes sorted4 through these tables: reject anything that
     // would leave [0, n)
+    int bad = 0;
     for (int h = 0; h < c->ncell; ++h) {
-        int b = cell_start_end[2 * h], e = cell_start_end[2 * h + 1];
-        if (b == -1) continue;
-        if (b < 0 || e < b || e > n) return PSIM_E_ARG;
+        const int b = cell_start_end[2 * h], e = cell_start_end[2 * h + 1];
+        bad |= (b != -1) & ((b < 0) | (e < b) | (e > n));
     }
     for (int i = 0; i < n; ++i) {
-        int o = hash_index[2 * i + 1];
-        if (o < 0 || o >= n) return PSIM_E_ARG;
+        const int o = hash_index[2 * i + 1];
+        bad |= (o < 0) | (o >= n);
     }
+    if (bad) return PSIM_E_ARG;
     int rc = 0;
     if (!c->tsorted) {
         if (!rc) rc = dalloc(&c->tsorted, 4 * (size_t)n);
@@ -867,12 +896,11 @@ int psim_gpu_force_table(psim_ctx *c, const double *sorted4, const int *hash_ind
         if (!rc) rc = dalloc(&c->tcse, 2 * (size_t)c->ncell);
         if (rc) return rc;
     }
-    CK(hipMemcpyAsync(c->tsorted, sorted4, sizeof(double) * 4 * n, hipMemcpyHostToDevice,
-                      c->stream));
-    CK(hipMemcpyAsync(c->thi, hash_index, sizeof(int) * 2 * n, hipMemcpyHostToDevice,
-                      c->stream));
-    CK(hipMemcpyAsync(c->tcse, cell_start_end, sizeof(int) * 2 * c->ncell,
-                      hipMemcpyHostToDevice, c->stream));
+    const Xfer x[3] = {{const_cast<double *>(sorted4), c->tsorted, sizeof(double) * 4 * (size_t)n},
+                       {const_cast<int *>(hash_index), c->thi, sizeof(int) * 2 * (size_t)n},
+                       {const_cast<int *>(cell_start_end), c->tcse,
+                        sizeof(int) * 2 * (size_t)c->ncell}};
+    if (stage_write(c->stage, c->stream, x, 3)) return PSIM_E_HIP;
     switch (c->pot.mask) {
     case 1: launch_table_mask<1>(c); break;
     case 2: launch_table_mask<2>(c); break;
@@ -884,12 +912,7 @@ int psim_gpu_force_table(psim_ctx *c, const double *sorted4, const int *hash_ind
     default: return PSIM_E_ARG;
     }
     CK(hipGetLastError());
-    CK(hipMemcpyAsync(force_out, c->fout, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
-                      c->stream));
-    CK(hipStreamSynchronize(c->stream));
-    int code = 0;
-    rc = read_error(c, &code, nullptr, nullptr);
-    return rc ? rc : code;
+    return read_forces(c, force_out);
 }
 
 int psim_gpu_pair_stats(psim_ctx *c, int which, int *count_by_orig,
@@ -910,12 +933,9 @@ int psim_gpu_pair_stats(psim_ctx *c, int which, int *count_by_orig,
     else
         psim::eng::launch_adj_stats(c, so);
     CK(hipGetLastError());
-    CK(hipMemcpyAsync(count_by_orig, c->st_count, sizeof(int) * n, hipMemcpyDeviceToHost,
-                      c->stream));
-    CK(hipMemcpyAsync(hash_by_orig, c->st_hash, sizeof(unsigned long long) * n,
-                      hipMemcpyDeviceToHost, c->stream));
-    CK(hipStreamSynchronize(c->stream));
-    return 0;
+    const Xfer x[2] = {{count_by_orig, c->st_count, sizeof(int) * (size_t)n},
+                       {hash_by_orig, c->st_hash, sizeof(unsigned long long) * (size_t)n}};
+    return stage_read(c->stage, c->stream, x, 2) ? PSIM_E_HIP : 0;
 }
 
 int psim_gpu_get_cells(psim_ctx *c, int *key_by_orig, int *cell_start, int *orig_by_slot)

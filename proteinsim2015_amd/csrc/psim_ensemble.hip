@@ -35,6 +35,7 @@
 #include "psim_build.hpp"
 #include "psim_gpu.h"
 #include "psim_params.hpp"
+#include "psim_stage.hpp"
 #include "psim_step.hpp"
 
 using namespace psim;
@@ -232,26 +233,36 @@ __global__ void k_iota_ens(int n, int *p)
     if (s < n) p[s] = s;
 }
 
-// The lagged arrays gathered into the current slot order (k_settle), pos0
-// (the positions the last step started from) re-imaged against pos in the
-// box of the slot's replica (slots p0[r]..p0[r+1] belong to replica r).
-__global__ void k_settle_ens(int n, const RepGeo *__restrict__ reps,
-                             const int *__restrict__ p0, int nrep,
-                             const int *__restrict__ prev, const double *__restrict__ pos0,
-                             const double *__restrict__ frc, const double *__restrict__ mem,
-                             const double *__restrict__ pos, double *__restrict__ pos0_out,
-                             double *__restrict__ frc_out, double *__restrict__ mem_out)
+// The state as n x 3 arrays by concatenated original index, the previous
+// positions and forces read where the last step left them (with prev, pos0
+// holds the positions it started from, re-imaged in the box of the slot's
+// replica).  Null outputs are skipped.
+__global__ void k_export_ens(int n, const RepGeo *__restrict__ reps, const int *__restrict__ p0,
+                             const int *__restrict__ rep_of, const int *__restrict__ id,
+                             const int *__restrict__ prev, const double *__restrict__ pos,
+                             const double *__restrict__ pos0, const double *__restrict__ vel,
+                             const double *__restrict__ frc, double *pos_out, double *pos0_out,
+                             double *vel_out, double *frc_out)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
-    const int p = prev[s];
-    const double L = reps[replica_of(p0, nrep, s)].g.L;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        pos0_out[d * n + s] = safe_mod0(pos0[d * n + p], pos[d * n + s], L);
-        frc_out[d * n + s] = frc[d * n + p];
-        mem_out[d * n + s] = mem[d * n + p];
+    const int o = id[s], p = prev ? prev[s] : s;
+    const double x = pos[s], y = pos[n + s], z = pos[2 * n + s];
+    if (pos_out) store_aos(pos_out, o, x, y, z);
+    if (pos0_out) {
+        double x0 = pos0[p], y0 = pos0[n + p], z0 = pos0[2 * n + p];
+        if (prev) {
+            int r = rep_of[s >> 8];
+            while (p0[r + 1] <= s) ++r;
+            const double L = reps[r].g.L;
+            x0 = safe_mod0(x0, x, L);
+            y0 = safe_mod0(y0, y, L);
+            z0 = safe_mod0(z0, z, L);
+        }
+        store_aos(pos0_out, o, x0, y0, z0);
     }
+    if (frc_out) store_aos(frc_out, o, frc[p], frc[n + p], frc[2 * n + p]);
+    if (vel_out) store_aos(vel_out, s, vel[s], vel[n + s], vel[2 * n + s]);   // by original index
 }
 
 // Initial hash of every particle into its replica's cells.
@@ -326,6 +337,7 @@ struct psim_ens {
     bool lagged = false;
     DevErr *err = nullptr;
     StepCtl *ctl = nullptr;
+    HostStage stage;   // pinned copies to the caller
     int *st_count = nullptr;                 // neighbour-set statistics
     unsigned long long *st_hash = nullptr;
     bool have_state = false;
@@ -458,24 +470,6 @@ void launch_build_ens(psim_ens *e, StepCtl *advance)
             e->upos, box);
     swap_lagged(e);
     e->lagged = true;
-}
-
-// The lagged arrays gathered into the current slot order, copied back so
-// that the buffers stay where a captured step sequence expects them.
-int settle_ens(psim_ens *e)
-{
-    if (!e->lagged) return 0;
-    const int n = e->ntot;
-    k_settle_ens<<<eblocks(n, 256), 256, 0, e->stream>>>(n, e->reps, e->p0, e->nrep, e->prev,
-                                                         e->pos0, e->frc, e->mem, e->pos,
-                                                         e->npos0, e->nfrc, e->nmem);
-    ECK(hipGetLastError());
-    const size_t b = sizeof(double) * 3 * (size_t)n;
-    ECK(hipMemcpyAsync(e->pos0, e->npos0, b, hipMemcpyDeviceToDevice, e->stream));
-    ECK(hipMemcpyAsync(e->frc, e->nfrc, b, hipMemcpyDeviceToDevice, e->stream));
-    ECK(hipMemcpyAsync(e->mem, e->nmem, b, hipMemcpyDeviceToDevice, e->stream));
-    e->lagged = false;
-    return 0;
 }
 
 // Workgroups of `block` lanes over the replicas `reps`.
@@ -740,6 +734,8 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
         rc = PSIM_E_HIP;
     if (!rc && hipMemset(e->count, 0, sizeof(int) * e->ncell) != hipSuccess) rc = PSIM_E_HIP;
     if (!rc && hipMemset(e->err, 0, sizeof(DevErr)) != hipSuccess) rc = PSIM_E_HIP;
+    // the four arrays of a state, each at an aligned place
+    if (!rc && !stage_reserve(e->stage, 4 * (sizeof(double) * n3 + 64))) rc = PSIM_E_HIP;
     if (rc) {
         psim_ens_destroy(e);
         return rc;
@@ -759,6 +755,7 @@ void psim_ens_destroy(psim_ens *e)
                     e->st_hash, e->prev, e->upos, e->rep_of};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    stage_free(e->stage);
     for (EnsClass &cl : e->cls) {   // the occupancy classes and the all-replica one
         void *cb[] = {cl.rmap, cl.wg, cl.item0};
         for (void *b : cb)
@@ -841,27 +838,24 @@ int psim_ens_get_state(psim_ens *e, double *pos, double *pos0, double *vel, doub
 {
     if (!e || !e->have_state) return PSIM_E_ARG;
     const int n = e->ntot;
-    int rs = settle_ens(e);
-    if (rs) return rs;
-    std::vector<int> ids(n);
-    std::vector<double> h(3 * (size_t)n);
-    ECK(hipStreamSynchronize(e->stream));
-    ECK(hipMemcpy(ids.data(), e->id, sizeof(int) * n, hipMemcpyDeviceToHost));
-    auto down = [&](const double *src, double *dst, bool by_slot) -> int {
-        if (!dst) return 0;
-        ECK(hipMemcpy(h.data(), src, sizeof(double) * 3 * n, hipMemcpyDeviceToHost));
-        for (int s = 0; s < n; ++s) {
-            const int o = by_slot ? ids[s] : s;
-            for (int d = 0; d < 3; ++d) dst[3 * (size_t)o + d] = h[(size_t)d * n + s];
-        }
-        return 0;
-    };
-    int rc;
-    if ((rc = down(e->pos, pos, true))) return rc;
-    if ((rc = down(e->pos0, pos0, true))) return rc;
-    if ((rc = down(e->vel, vel, false))) return rc;
-    if ((rc = down(e->frc, frc, true))) return rc;
-    return 0;
+    // n x 3 arrays made on the device in buffers that hold nothing between
+    // steps, then copied out through pinned memory
+    double *dst[4] = {pos, pos0, vel, frc};
+    double *out[4] = {e->npos, e->npos0, e->nmem, e->nfrc};
+    const size_t b = sizeof(double) * 3 * (size_t)n;
+    Xfer x[4];
+    int nx = 0;
+    for (int k = 0; k < 4; ++k) {
+        if (dst[k])
+            x[nx++] = Xfer{dst[k], out[k], b};
+        else
+            out[k] = nullptr;
+    }
+    k_export_ens<<<eblocks(n, 256), 256, 0, e->stream>>>(
+        n, e->reps, e->p0, e->rep_of, e->id, e->lagged ? e->prev : nullptr, e->pos, e->pos0,
+        e->vel, e->frc, out[0], out[1], out[2], out[3]);
+    ECK(hipGetLastError());
+    return stage_read(e->stage, e->stream, x, nx) ? PSIM_E_HIP : 0;
 }
 
 int psim_ens_set_graph(psim_ens *e, int steps_per_graph)
@@ -902,8 +896,8 @@ int psim_ens_last_error(psim_ens *e, int *code, int *i, int *j)
 {
     if (!e) return PSIM_E_ARG;
     DevErr h{};
-    ECK(hipStreamSynchronize(e->stream));
-    ECK(hipMemcpy(&h, e->err, sizeof(h), hipMemcpyDeviceToHost));
+    const Xfer x{&h, e->err, sizeof(h)};
+    if (stage_read(e->stage, e->stream, &x, 1)) return PSIM_E_HIP;
     if (code) *code = h.code;
     if (i) *i = h.i;
     if (j) *j = h.j;
@@ -944,12 +938,9 @@ int psim_ens_pair_stats(psim_ens *e, int *count_by_orig, unsigned long long *has
 #undef PSIM_ENS_STATS
     }
     ECK(hipGetLastError());
-    ECK(hipMemcpyAsync(count_by_orig, e->st_count, sizeof(int) * n, hipMemcpyDeviceToHost,
-                       e->stream));
-    ECK(hipMemcpyAsync(hash_by_orig, e->st_hash, sizeof(unsigned long long) * n,
-                       hipMemcpyDeviceToHost, e->stream));
-    ECK(hipStreamSynchronize(e->stream));
-    return 0;
+    const Xfer x[2] = {{count_by_orig, e->st_count, sizeof(int) * (size_t)n},
+                       {hash_by_orig, e->st_hash, sizeof(unsigned long long) * (size_t)n}};
+    return stage_read(e->stage, e->stream, x, 2) ? PSIM_E_HIP : 0;
 }
 
 // For each occupancy class, and for all replicas as one launch: time every

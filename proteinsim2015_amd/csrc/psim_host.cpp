@@ -11,11 +11,38 @@
 //     against the points accepted earlier in the same round.
 // The result is exactly sequential addition over the candidate stream, so it
 // does not depend on the thread count.
+#include <omp.h>
+
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <cstring>
 #include <vector>
 
 #include "psim_gpu.h"
+
+namespace psim {
+
+// memcpy for arrays that arrive in staging memory: from 1 MiB on, a few
+// threads share the copy and the page faults of a fresh destination (48 MB
+// into fresh pages: 3.8 ms on one thread).
+void host_copy(void *dst, const void *src, size_t bytes)
+{
+    constexpr size_t kPart = 128u << 10;
+    const long parts = (long)((bytes + kPart - 1) / kPart);
+    const int threads = std::min({8, omp_get_max_threads(), (int)(bytes >> 19)});
+    if (threads < 2) {
+        std::memcpy(dst, src, bytes);
+        return;
+    }
+#pragma omp parallel for schedule(static) num_threads(threads)
+    for (long k = 0; k < parts; ++k) {
+        const size_t off = (size_t)k * kPart;
+        std::memcpy((char *)dst + off, (const char *)src + off, std::min(kPart, bytes - off));
+    }
+}
+
+}  // namespace psim
 
 namespace {
 

@@ -137,7 +137,7 @@ void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot, con
     if (path.dense) {
         const int per = (geo.ncell + 7) / 8;
         auto launch = [&](auto ljn) {
-            k_forces_dense<MASK, decltype(ljn)::value, true>
+            k_forces_dense<MASK, decltype(ljn)::value>
                 <<<8 * per, kDenseThreads, 0, st>>>(geo, pot, P.radius, pos, id, cstart, fout,
                                                     err, per);
         };
@@ -153,17 +153,17 @@ void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot, con
     } else if (path.brick) {
         const int per = (path.bg.nbricks + 7) / 8;
         if (path.brick_g == 1)
-            k_forces_brick<MASK, 1, true><<<8 * per, kBrickThreads, 0, st>>>(
+            k_forces_brick<MASK, 1><<<8 * per, kBrickThreads, 0, st>>>(
                 geo, pot, P.radius, path.bg, per, pos, id, cstart, fout, err);
         else
-            k_forces_brick<MASK, kSmallSplit, true><<<8 * per, kBrickThreads, 0, st>>>(
+            k_forces_brick<MASK, kSmallSplit><<<8 * per, kBrickThreads, 0, st>>>(
                 geo, pot, P.radius, path.bg, per, pos, id, cstart, fout, err);
     } else if (n < kSmallSystem) {
-        k_forces<MASK, 64, kSmallSplit, true>
+        k_forces<MASK, 64, kSmallSplit>
             <<<xcd_grid(eng::blocks_for((long long)n * kSmallSplit, 64)), 64, 0, st>>>(
                 geo, pot, cull, P.radius, pos, upos, id, cstart, fout, err);
     } else {
-        k_forces<MASK, kBlock, 1, true>
+        k_forces<MASK, kBlock, 1>
             <<<xcd_grid(eng::blocks_for(n, kBlock)), kBlock, 0, st>>>(
                 geo, pot, cull, P.radius, pos, upos, id, cstart, fout, err);
     }

@@ -10,6 +10,7 @@
 #include "psim_gather.hpp"
 #include "psim_gpu.h"
 #include "psim_pairs.hpp"
+#include "psim_stage.hpp"
 
 namespace psim {
 namespace {
@@ -320,25 +321,8 @@ __global__ __launch_bounds__(256) void k_integrate(Geo g, GB gb, StepArgs a)
     integrate_one<false>(g, gb, a, s, a.nfrc[s], a.nfrc[N + s], a.nfrc[2 * N + s]);
 }
 
-// The force on the particle of original index o, by original index: [3][N]
-// (SoA) or, with AOS, N x 3.
-template <bool AOS>
-__device__ __forceinline__ void store_force(double *fout, int N, int o, double fx, double fy,
-                                            double fz)
-{
-    if (AOS) {
-        fout[3 * (size_t)o] = fx;
-        fout[3 * (size_t)o + 1] = fy;
-        fout[3 * (size_t)o + 2] = fz;
-    } else {
-        fout[o] = fx;
-        fout[N + o] = fy;
-        fout[2 * N + o] = fz;
-    }
-}
-
-// Forces only at the current state, written by original index.
-template <int MASK, int BLOCK, int SPLIT, bool AOS = false>
+// Forces only at the current state, written by original index (N x 3).
+template <int MASK, int BLOCK, int SPLIT>
 __global__ __launch_bounds__(BLOCK) void k_forces(Geo g, Pot p, Cull q, double radius,
                                                    const double *pos, const uint4 *upos,
                                                    const int *id, const int *cstart,
@@ -358,11 +342,11 @@ __global__ __launch_bounds__(BLOCK) void k_forces(Geo g, Pot p, Cull q, double r
     fx = split_sum<SPLIT>(fx);
     fy = split_sum<SPLIT>(fy);
     fz = split_sum<SPLIT>(fz);
-    if (sub == 0 && valid) store_force<AOS>(fout, N, id[s], fx, fy, fz);
+    if (sub == 0 && valid) store_aos(fout, id[s], fx, fy, fz);
 }
 
 // Forces only, brick per workgroup (same result as k_forces with SPLIT = G).
-template <int MASK, int G, bool AOS = false>
+template <int MASK, int G>
 __global__ __launch_bounds__(kBrickThreads) void k_forces_brick(Geo g, Pot p, double radius,
                                                                 BrickGeo bg, int per_xcd,
                                                                 const double *pos,
@@ -373,9 +357,8 @@ __global__ __launch_bounds__(kBrickThreads) void k_forces_brick(Geo g, Pot p, do
     __shared__ BrickShared sh;
     const int b = xcd_cell(blockIdx.x, per_xcd);
     if (b >= bg.nbricks) return;
-    const int N = g.n;
     auto epi = [&](int s, double fx, double fy, double fz) {
-        store_force<AOS>(fout, N, id[s], fx, fy, fz);
+        store_aos(fout, id[s], fx, fy, fz);
     };
     if (g.exact_mi)
         brick_forces<MASK, true, G>(g, p, radius, pos, cstart, id, err, bg, b, sh, epi);
@@ -383,7 +366,7 @@ __global__ __launch_bounds__(kBrickThreads) void k_forces_brick(Geo g, Pot p, do
         brick_forces<MASK, false, G>(g, p, radius, pos, cstart, id, err, bg, b, sh, epi);
 }
 
-template <int MASK, int LJN, bool AOS = false>
+template <int MASK, int LJN>
 __global__ __launch_bounds__(kDenseThreads)
 __attribute__((amdgpu_waves_per_eu(dense_waves(MASK, LJN)))) void k_forces_dense(
     Geo g, Pot p, double radius, const double *pos, const int *id, const int *cstart,
@@ -393,10 +376,9 @@ __attribute__((amdgpu_waves_per_eu(dense_waves(MASK, LJN)))) void k_forces_dense
     const int c = xcd_cell(blockIdx.x, per_xcd);
     if (c >= g.ncell) return;
     const int home0 = cstart[c];
-    const int N = g.n;
     dense_cell_forces<MASK, kDenseThreads, LJN>(g, p, radius, pos, cstart, id, err, c, sh,
                             [=](int i, double Fx, double Fy, double Fz) {
-                                store_force<AOS>(fout, N, id[home0 + i], Fx, Fy, Fz);
+                                store_aos(fout, id[home0 + i], Fx, Fy, Fz);
                             });
 }
 
@@ -499,9 +481,7 @@ __global__ __launch_bounds__(BLOCK) void k_forces_table(Geo g, Pot p, Cull q, co
     fz = split_sum<SPLIT>(fz);
     if (sub != 0 || !valid) return;
     const int o = orig(s);
-    fout[3 * (size_t)o] = fx;   // particleForce[3*orig + k] (LJPotential.cpp:179-181)
-    fout[3 * (size_t)o + 1] = fy;
-    fout[3 * (size_t)o + 2] = fz;
+    store_aos(fout, o, fx, fy, fz);   // particleForce[3*orig + k] (LJPotential.cpp:179-181)
 }
 
 
