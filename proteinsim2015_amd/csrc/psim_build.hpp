@@ -4,13 +4,16 @@
 //
 // Replaces system::hashParticles / sortParticles / clearCells /
 // reorderParticles (systemHandling.cpp:33-85): instead of an O(N log N)
-// comparison sort of (hash, index) tuples every step, each particle's new
-// cell is counted with a wave-aggregated atomic during the step, the counts
-// are scanned into a start table, and the state is gathered into cell order.
-// Within a cell the order is the previous slot order (a stable counting
-// sort), which makes every run reproducible bit for bit.
+// comparison sort of (hash, index) tuples every step, each particle is
+// entered in the bin of its new cell during the step, and one kernel turns
+// the bins into a start table and moves the state into cell order.  Within a
+// cell the order is the previous slot order (a stable counting sort), which
+// makes every run reproducible bit for bit.  The scan and scatter kernels
+// below serve the rebuilds that start from counts (analysis grid, forces
+// without a context).
 #pragma once
 
+#include "psim_bins.hpp"
 #include "psim_gather.hpp"
 
 namespace psim {
@@ -20,7 +23,18 @@ constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
-// Cell hash + atomic count for an arbitrary order (initial build).
+// Every particle into its cell's bin, in an arbitrary order (initial build).
+__global__ void k_bin_all(Geo g, const double *pos, Bins b)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= g.n) return;
+    const int N = g.n;
+    const int k = g.c0 + cell_1d(pos[s], g.cell, g.S) + g.S * cell_1d(pos[N + s], g.cell, g.S)
+                + g.S2 * cell_1d(pos[2 * N + s], g.cell, g.S);
+    bin_particle(b, N, s, k);
+}
+
+// Cell hash + atomic count for an arbitrary order.
 __global__ void k_hash_count(Geo g, const double *pos, int *key, int *arank, int *count)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -114,15 +128,13 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_bsum(int *bsum, int nb)
 }
 
 // Cell start table from the counts: block b scans its tile on top of the
-// prefix of the tile totals before it, writes the starts (also to cstart2
-// when set) and clears the counts for the next step's counting.  With
+// prefix of the tile totals before it, writes the starts and clears the counts for the next step's counting.  With
 // RESUM, the block sums the raw totals bsum[0..b) itself (few tiles);
 // otherwise bsum already holds the prefixes (k_scan_bsum).
 template <bool RESUM>
 __global__ __launch_bounds__(kScanThreads) void k_scan_apply(int *count, int ncell,
                                                              const int *bsum,
-                                                             int *cstart, int n,
-                                                             int *cstart2)
+                                                             int *cstart, int n)
 {
     int before;
     if constexpr (RESUM) {
@@ -140,23 +152,18 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(int *count, int nce
     if (base + kScanItems <= ncell) {
         const int4 st = make_int4(pre, pre + c[0], pre + c[0] + c[1], pre + c[0] + c[1] + c[2]);
         *reinterpret_cast<int4 *>(cstart + base) = st;
-        if (cstart2) *reinterpret_cast<int4 *>(cstart2 + base) = st;
         *reinterpret_cast<int4 *>(count + base) = make_int4(0, 0, 0, 0);
     } else {
 #pragma unroll
         for (int k = 0; k < kScanItems; ++k) {
             if (base + k < ncell) {
                 cstart[base + k] = pre;
-                if (cstart2) cstart2[base + k] = pre;
                 count[base + k] = 0;
             }
             pre += c[k];
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        cstart[ncell] = n;
-        if (cstart2) cstart2[ncell] = n;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) cstart[ncell] = n;
 }
 
 // The scan of the cell counts into the start table for grids of more than
@@ -166,16 +173,14 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(int *count, int nce
 // (three launches; the re-summing grows with the square of the tile count).
 constexpr int kScanResumTiles = 256;
 inline void launch_scan3(hipStream_t st, int *count, int ncell, int nscan, int *bsum,
-                         int *cstart, int n, int *cstart2 = nullptr)
+                         int *cstart, int n)
 {
     k_scan_reduce<<<nscan, kScanThreads, 0, st>>>(count, ncell, bsum);
     if (nscan <= kScanResumTiles) {
-        k_scan_apply<true><<<nscan, kScanThreads, 0, st>>>(count, ncell, bsum, cstart, n,
-                                                           cstart2);
+        k_scan_apply<true><<<nscan, kScanThreads, 0, st>>>(count, ncell, bsum, cstart, n);
     } else {
         k_scan_bsum<<<1, kScanThreads, 0, st>>>(bsum, nscan);
-        k_scan_apply<false><<<nscan, kScanThreads, 0, st>>>(count, ncell, bsum, cstart, n,
-                                                            cstart2);
+        k_scan_apply<false><<<nscan, kScanThreads, 0, st>>>(count, ncell, bsum, cstart, n);
     }
 }
 
@@ -189,8 +194,7 @@ inline void launch_scan3(hipStream_t st, int *count, int ncell, int nscan, int *
 // direct form is kept for the smallest grids only)
 constexpr int kScanDirectTiles = 4;
 __global__ __launch_bounds__(kScanThreads) void k_scan_direct(const int *count, int ncell,
-                                                              int *cstart, int n,
-                                                              int *cstart2 = nullptr)
+                                                              int *cstart, int n)
 {
     const int lim = blockIdx.x * kScanTile;   // a multiple of 4, at most ncell
     int before = 0;
@@ -221,69 +225,24 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_direct(const int *count, 
     int pre = block_exclusive_scan(v, &total) + before_total;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
-        if (base + k < ncell) {
-            cstart[base + k] = pre;
-            if (cstart2) cstart2[base + k] = pre;
-        }
+        if (base + k < ncell) cstart[base + k] = pre;
         pre += c[k];
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        cstart[ncell] = n;
-        if (cstart2) cstart2[ncell] = n;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) cstart[ncell] = n;
 }
 
 // With clear_count set (after k_scan_direct), also zeroes the ncell counts
-// for the next step's counting.  Each lane places U slots (s, s + blockDim.x,
-// ... of its block's U * blockDim.x), their loads issued together.
-template <int U = 1>
+// for the next call's counting.
 __global__ __launch_bounds__(256) void k_scatter(int n, const int *key, const int *arank,
                                                  const int *cstart, int *perm,
                                                  int *clear_count, int ncell)
 {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (clear_count)
-        for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell;
-             c += gridDim.x * blockDim.x)
-            clear_count[c] = 0;
-    const int s0 = blockIdx.x * (blockDim.x * U) + threadIdx.x;
-    int k[U], r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int s = s0 + u * (int)blockDim.x;
-        k[u] = s < n ? key[s] : 0;
-        r[u] = s < n ? arank[s] : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int s = s0 + u * (int)blockDim.x;
-        if (s < n) perm[cstart[k[u]] + r[u]] = s;
-    }
+        for (int c = s; c < ncell; c += gridDim.x * blockDim.x) clear_count[c] = 0;
+    if (s < n) perm[cstart[key[s]] + arank[s]] = s;
 }
 
-// Canonical order within a cell = ascending source slot (a stable counting
-// sort).  Only the positions and the original ids are gathered into the new
-// order; prev[dst] records the slot each particle came from, so the
-// integrator reads the previous positions, forces and memory of the last
-// step where it wrote them (at prev[s]) instead of every array moving every
-// step.
-// With ctl set (a step sequence whose control lives in device memory), the
-// kernel also ends the step: it advances the clock and the next step's
-// flags, which no kernel of this step reads after the integrator.  With
-// pos2 / id2 set, the new positions and ids are also written there (a
-// record of the state, e.g. the adjoint's recomputed trajectory), and with
-// inv2 the slot of each original index.
-//
-// Each lane moves U particles (slots t, t + blockDim.x, ... of its block's
-// U * blockDim.x), their loads interleaved: the kernel is bound by the
-// latency of its chain of dependent gathers (slot -> particle -> cell ->
-// the cell's members), not by its bytes.
-#ifndef PSIM_MOVE_ILP
-#define PSIM_MOVE_ILP 4
-#endif
-constexpr int kMoveIlp = PSIM_MOVE_ILP;
-// below this many particles the grid is too small to give up lanes for
-// interleaving (one particle per lane)
-constexpr int kMoveIlpMin = 1 << 20;
 // 1 / L of the box that slot t's particle lives in: one box for all; NoBox
 // where the pair kernel reads no box fractions.
 struct OneBox {
@@ -295,71 +254,264 @@ struct NoBox {
     static constexpr bool kPack = false;
     __device__ double operator()(int) const { return 0.0; }
 };
-// Box::kPack: the new positions' box fractions and cells are written to upos
-// too (the thread-per-particle kernels' cull).
+
+// Where the rebuild writes the new order.  With cstart2 / pos2 / id2 set, the
+// cell table and the new positions and ids are also written there (a record
+// of the state, e.g. the adjoint's recomputed trajectory), and with inv2 the
+// slot of each original index.
+struct Rebuilt {
+    int *cstart;
+    double *pos;
+    int *id, *prev;
+    uint4 *upos;
+    int *cstart2;
+    double *pos2;
+    int *id2, *inv2;
+};
+
+constexpr int kTileThreads = 256;
+
+// The cell rebuild in one launch: start table, canonical order, positions and
+// ids moved into it.
+//
+// A workgroup owns a tile of 1 << shift consecutive cells.  Its first slot is
+// the sum of the tile totals before it (prefixed: tile_total already holds
+// that sum), the starts of its cells a scan of their counts; the members come
+// from the cells' bins, and a member's place in its cell is the number of
+// members with a lower slot.  Canonical order within a cell = ascending
+// source slot (a stable counting sort).  Only the positions and the original
+// ids are gathered into the new order; prev[dst] records the slot each
+// particle came from, so the integrator reads the previous positions, forces
+// and memory of the last step where it wrote them (at prev[s]) instead of
+// every array moving every step.
+//
+// Bound by latency: three dependent rounds of loads (counts and totals, bins,
+// positions) and one of stores.  As separate kernels (counts summed by tile,
+// start table, scatter into cell order, move) it was nine such rounds and
+// three more launch boundaries: 4.9 + 5.4 + 4.7 + 6.6 us of a 45 us step at
+// 262,144 AO particles, now a step of 33.3; 19.1 for 23.0 us at 4,096 (three
+// kernels before), 27.4 for 36.0 at 30,011, 829 for 900 at 2,097,152.
+//
+// Each lane moves up to U particles with their loads together; a tile with
+// more members than U * kTileThreads keeps its list in perm (which has room
+// for it at the tile's slots) instead of LDS and goes round by round.
+//
+// The kernel clears what the next step counts into: the counts of its cells,
+// the heads of its chains, and next_total, the other of two arrays of tile
+// totals (this step's are still being read).  With ctl set (a step sequence
+// whose control lives in device memory) it also ends the step: it advances
+// the clock and the next step's flags, which no kernel of this step reads
+// after the integrator.  Box::kPack: the new positions' box fractions and
+// cells are written to upos too (the thread-per-particle kernels' cull).
 template <int U, class Box>
-__global__ __launch_bounds__(256) void k_move_lagged(
-    int n, const int *__restrict__ perm, const int *__restrict__ key,
-    const int *__restrict__ cstart, const double *__restrict__ npos,
-    const int *__restrict__ id_in, double *__restrict__ pos, int *__restrict__ id_out,
-    int *__restrict__ prev, StepCtl *ctl, uint4 *__restrict__ upos, Box box,
-    double *__restrict__ pos2 = nullptr, int *__restrict__ id2 = nullptr,
-    int *__restrict__ inv2 = nullptr)
+__global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins b, int prefixed,
+                                                          int *next_total, int *perm,
+                                                          const double *__restrict__ npos,
+                                                          const int *__restrict__ id_in,
+                                                          StepCtl *ctl, Box box, Rebuilt to)
 {
-    const int t0 = blockIdx.x * (blockDim.x * U) + threadIdx.x;
-    if (ctl && t0 == 0) ctl_advance(ctl);
-    if (t0 >= n) return;
-    int s[U], c[U], b[U], len[U], rank[U];
-    double inv_L[U];
-    bool ok[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int t = t0 + u * (int)blockDim.x;
-        ok[u] = t < n;
-        s[u] = perm[ok[u] ? t : t0];   // a missing slot repeats the first
-        if (Box::kPack) inv_L[u] = box(ok[u] ? t : t0);   // the box of the slot's cell
+    constexpr int kList = U * kTileThreads;
+    __shared__ int start[kTileCells + 1];
+    __shared__ int list[kList];
+    __shared__ unsigned short cell_of[kList];
+    __shared__ int wsum[2][kTileThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    // below the size of U = 4 a tile runs on the XCD whose L2 the integrator
+    // left its particles in (xcd_block's order; 34.0 -> 33.3 us a step at
+    // 262,144 particles, 7.25 -> 7.07 ms a fit at 32,768; at 2,097,152 they
+    // are long gone, and the launch order is 3 us faster)
+    const int tile = U < 4 ? xcd_block() : blockIdx.x;
+    if (U < 4 && ((long long)tile << b.shift) >= ncell) return;
+    const int c0 = tile << b.shift;
+    const int cells = min(1 << b.shift, ncell - c0);
+    if (ctl && tile == 0 && tid == 0) ctl_advance(ctl);
+
+    // totals of the tiles before this one; this lane's four counts
+    int before = 0;
+    if (prefixed) {
+        if (tid == 0) before = b.tile_total[tile];
+    } else {
+        for (int i = tid * 4; i < tile; i += kTileThreads * 4) {
+            const int4 q = *reinterpret_cast<const int4 *>(b.tile_total + i);
+            before += q.x + (i + 1 < tile ? q.y : 0) + (i + 2 < tile ? q.z : 0) +
+                      (i + 3 < tile ? q.w : 0);
+        }
     }
-    int most = 0;
+    const int k0 = tid * 4;
+    int cnt[4] = {0, 0, 0, 0};
+    if (k0 + 4 <= cells) {
+        int4 *p = reinterpret_cast<int4 *>(b.count + c0 + k0);
+        const int4 q = *p;
+        cnt[0] = q.x;
+        cnt[1] = q.y;
+        cnt[2] = q.z;
+        cnt[3] = q.w;
+        *p = make_int4(0, 0, 0, 0);
+    } else {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-        c[u] = key[s[u]];
-        b[u] = cstart[c[u]];
-        len[u] = cstart[c[u] + 1] - b[u];
-        rank[u] = 0;
-        most = max(most, len[u]);
+        for (int k = 0; k < 4; ++k)
+            if (k0 + k < cells) {
+                cnt[k] = b.count[c0 + k0 + k];
+                b.count[c0 + k0 + k] = 0;
+            }
     }
-    // rank among the cell's members: four independent loads per particle
-    // per round
-    for (int k = 0; k < most; k += 4) {
+    if (tid == 0) next_total[tile] = 0;
+    const int mine = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    int x = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+        before += __shfl_xor(before, d, 64);
+    }
+    if (lane == 63) {
+        wsum[0][w] = x;
+        wsum[1][w] = before;
+    }
+    __syncthreads();
+    int pre = x - mine, base = 0, m = 0;
+#pragma unroll
+    for (int v = 0; v < kTileThreads / 64; ++v) {
+        if (v < w) pre += wsum[0][v];
+        m += wsum[0][v];
+        base += wsum[1][v];
+    }
+    const bool fits = m <= kList;
+    {
+        const int st[4] = {pre, pre + cnt[0], pre + cnt[0] + cnt[1], pre + cnt[0] + cnt[1] + cnt[2]};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k0 + k < cells) {
+                start[k0 + k] = st[k];
+                if (fits)
+                    for (int j = 0; j < cnt[k]; ++j) cell_of[st[k] + j] = (unsigned short)(k0 + k);
+            }
+        if (k0 + 4 <= cells) {
+            const int4 q = make_int4(base + st[0], base + st[1], base + st[2], base + st[3]);
+            *reinterpret_cast<int4 *>(to.cstart + c0 + k0) = q;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k0 + k < cells) to.cstart[c0 + k0 + k] = base + st[k];
+        }
+        if (to.cstart2) {   // of any alignment
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k0 + k < cells) to.cstart2[c0 + k0 + k] = base + st[k];
+        }
+    }
+    if (tid == 0) {
+        start[cells] = m;
+        if (c0 + cells == ncell) {
+            to.cstart[ncell] = n;
+            if (to.cstart2) to.cstart2[ncell] = n;
+        }
+    }
+    __syncthreads();
+    if (m == 0) return;
+
+    // member j of the tile (cell i, r-th of its bin) into the list; the first
+    // member past the row walks the cell's chain
+    auto fetch = [&](int j, int i, int *out) {
+        const int r = j - start[i];
+        const int c = c0 + i;
+        if (r < b.cap) {
+            const int s = b.tab[(size_t)c * b.cap + r];
+            out[j] = s;
+            return s;
+        }
+        if (r == b.cap) {
+            int *head = b.over + (size_t)n + c;
+            int s = *head;
+            *head = -1;
+            for (int q = j; q < start[i + 1] && s >= 0; ++q) {
+                out[q] = s;
+                s = b.over[s];
+            }
+        }
+        return -1;
+    };
+    auto place = [&](int i, int rank, int s, double px, double py, double pz, int o) {
+        const int dst = base + start[i] + rank;
+        to.pos[dst] = px;
+        to.pos[n + dst] = py;
+        to.pos[2 * n + dst] = pz;
+        if (to.pos2) {
+            to.pos2[dst] = px;
+            to.pos2[n + dst] = py;
+            to.pos2[2 * n + dst] = pz;
+        }
+        if (Box::kPack) to.upos[dst] = pack_position(px, py, pz, c0 + i, box(dst));
+        to.id[dst] = o;
+        if (to.id2) to.id2[dst] = o;
+        if (to.inv2) to.inv2[o] = dst;
+        to.prev[dst] = s;
+    };
+    auto rank_in = [&](const int *l, int i, int s) {
+        int rank = 0;
+        for (int k = start[i]; k < start[i + 1]; ++k) rank += l[k] < s;
+        return rank;
+    };
+    if (fits) {
+        int i[U], s[U], o[U];
+        double p[U][3];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+            const int j = tid + u * kTileThreads;
+            i[u] = j < m ? cell_of[j] : 0;
+            s[u] = j < m ? fetch(j, i[u], list) : -1;
+        }
+        __syncthreads();
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (k + q < len[u]) rank[u] += (perm[b[u] + k + q] < s[u]);
+        for (int u = 0; u < U; ++u) {
+            const int j = tid + u * kTileThreads;
+            if (s[u] < 0) s[u] = j < m ? list[j] : list[0];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) p[u][d] = npos[d * n + s[u]];
+            o[u] = id_in[s[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (tid + u * kTileThreads < m)
+                place(i[u], rank_in(list, i[u], s[u]), s[u], p[u][0], p[u][1], p[u][2], o[u]);
+    } else {
+        auto cell = [&](int j) {   // the last cell that starts at or before j
+            int lo = 0, hi = cells - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (start[mid] <= j) lo = mid; else hi = mid - 1;
+            }
+            return lo;
+        };
+        int *l = perm + base;
+        for (int j = tid; j < m; j += kTileThreads) fetch(j, cell(j), l);
+        __syncthreads();
+        for (int j = tid; j < m; j += kTileThreads) {
+            const int s = l[j], i = cell(j);
+            place(i, rank_in(l, i, s), s, npos[s], npos[n + s], npos[2 * n + s], id_in[s]);
         }
     }
-    double x[U][3];
-    int o[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) x[u][d] = npos[d * n + s[u]];
-        o[u] = id_in[s[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        if (!ok[u]) continue;
-        const int dst = b[u] + rank[u];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            pos[d * n + dst] = x[u][d];
-            if (pos2) pos2[d * n + dst] = x[u][d];
-        }
-        if (Box::kPack) upos[dst] = pack_position(x[u][0], x[u][1], x[u][2], c[u], inv_L[u]);
-        id_out[dst] = o[u];
-        if (id2) id2[dst] = o[u];
-        if (inv2) inv2[o[u]] = dst;
-        prev[dst] = s[u];
+}
+
+// A workgroup sums the totals before its tile itself up to this many tiles
+// (eight loads of 16 bytes per lane); beyond that one block turns them into
+// prefixes first.
+constexpr int kSelfPrefixTiles = 8192;
+
+template <class Box>
+void launch_rebuild(hipStream_t st, int n, int ncell, BinStore &t, const double *npos,
+                    const int *id_in, StepCtl *ctl, Box box, const Rebuilt &to)
+{
+    const int prefixed = t.tiles > kSelfPrefixTiles;
+    if (prefixed) k_scan_bsum<<<1, kScanThreads, 0, st>>>(t.b.tile_total, t.tiles);
+    auto go = [&](auto u) {
+        k_rebuild<decltype(u)::value><<<decltype(u)::value < 4 ? xcd_grid(t.tiles) : t.tiles, kTileThreads, 0, st>>>(
+            n, ncell, t.b, prefixed, t.next_total, t.perm, npos, id_in, ctl, box, to);
+    };
+    switch (t.lanes) {
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    default: go(std::integral_constant<int, 1>{}); break;
     }
 }
 

@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <vector>
 
+#include "psim_bins.hpp"
 #include "psim_brick_shape.hpp"
 #include "psim_device.hpp"
 #include "psim_gpu.h"
@@ -14,7 +15,7 @@
 
 // The buffers and constants a captured step sequence bakes into its kernels.
 struct GraphKey {
-    const void *pos, *pos0, *frc, *mem, *npos, *npos0, *nfrc, *nmem, *id, *nid, *pbc;
+    const void *pos, *pos0, *frc, *mem, *npos, *npos0, *nfrc, *nmem, *id, *nid, *pbc, *totals;
     psim::Geo geo;
     psim::Pot pot;
     psim::GB gb;
@@ -30,7 +31,7 @@ struct psim_ctx {
     psim::Pot pot;
     psim::GB gb;
     psim::Cull cull;   // derived from geo and pot
-    int n = 0, ncell = 0, nscan = 0;
+    int n = 0, ncell = 0;
     bool dense = false;   // cell-per-workgroup pair kernel (else thread per particle)
     bool brick = false;   // brick-per-workgroup pair kernel (sparse systems)
     psim::BrickGeo bg{};  // its bricks
@@ -41,7 +42,7 @@ struct psim_ctx {
     double *vel = nullptr, *fout = nullptr;
     uint4 *upos = nullptr;   // box fractions and cells of pos, in its slot order
                              // (thread-per-particle path only)
-    int *id = nullptr, *nid = nullptr, *key = nullptr, *arank = nullptr, *perm = nullptr;
+    int *id = nullptr, *nid = nullptr;
     // pos0 / frc / mem stay in the slot order of the last step: pos0 the
     // positions that step started from (not yet re-imaged), frc and mem what
     // it wrote; prev[s] is the slot in that order of the particle now in
@@ -56,7 +57,8 @@ struct psim_ctx {
     hipGraphExec_t gexec = nullptr;
     GraphKey gkey{};
     psim::StepCtl *ctl = nullptr;
-    int *count = nullptr, *cstart = nullptr, *bsum = nullptr;
+    int *cstart = nullptr;
+    psim::BinStore bins;        // members of the cells after the step
     psim::DevErr *err = nullptr;
     double *noise = nullptr;
     size_t noise_cap = 0;

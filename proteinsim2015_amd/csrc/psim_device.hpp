@@ -408,6 +408,41 @@ __device__ __forceinline__ int wave_aggregated_rank(int *count, int key)
     return base + __popcll(active & le & ~((1ull << leader) - 1ull)) - 1;
 }
 
+// tile_total[t] += 1 for every active lane, one atomic per distinct t of the
+// wave (the particles of a wave sit in a few consecutive tiles).
+__device__ __forceinline__ void wave_count(int *tile_total, int t)
+{
+    const int lane = (int)__lane_id();
+    unsigned long long todo = __ballot(1);
+    while (todo) {
+        const int leader = __ffsll((long long)todo) - 1;
+        const unsigned long long same = __ballot(t == __builtin_amdgcn_readlane(t, leader));
+        if (lane == leader) atomicAdd(&tile_total[t], __popcll(same & todo));
+        todo &= ~same;
+    }
+}
+
+// What a step's integrator leaves for the cell rebuild: the members of every
+// cell in any order and the totals of the tiles of 1 << shift cells.
+struct Bins {
+    int *count;        // [cells] members; the rebuild clears it
+    int *tab;          // [cells][cap] slots of the first cap members
+    int *over;         // [n] next, [cells] head: the members past cap as chains
+    int *tile_total;   // [tiles]
+    int cap, shift;
+};
+
+// The particle of slot s goes to cell c (n particles in all).
+__device__ __forceinline__ void bin_particle(const Bins &b, int n, int s, int c)
+{
+    wave_count(b.tile_total, c >> b.shift);
+    const int r = wave_aggregated_rank(b.count, c);
+    if (r < b.cap)
+        b.tab[(size_t)c * b.cap + r] = s;
+    else
+        b.over[s] = atomicExch(&b.over[(size_t)n + c], s);
+}
+
 // ---------------------------------------------------------------------------
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11) and Box-Muller normals.
 // counter = (id, step_lo, step_hi, block), key = (seed_lo, seed_hi).

@@ -12,20 +12,15 @@
 // One step (the order of system::run, system.cpp:187-211):
 //   k_step      fused: 27-cell forces F(x_n) (IForce::getAcceleration),
 //               push (frc0 <- frc), G&B integration (firstStep/normalStep/
-//               velocityStep), wrap (particle::setPos), new cell hash and
-//               an atomic per-cell count; writes the next state in the
-//               current slot order to the "n*" buffers.
-//   k_scan_*    counts -> cstart (exclusive scan), counts cleared: tile
-//               totals, their prefix (one block), then each tile's scan;
-//               one launch, k_scan_direct, for grids of up to 32 scan
-//               tiles (k_scatter then clears the counts).
-//   k_scatter   slot of each particle in its new cell (arbitrary order).
-//   k_move_lagged  canonical within-cell order (ascending previous slot,
-//               i.e. a stable counting sort); positions and ids move into
-//               it; the positions the step started from (pos0 of the next
-//               step, re-imaged when read), the forces and the memory stay
-//               where the step had or wrote them (read through the slot map
-//               prev).
+//               velocityStep), wrap (particle::setPos), entry in the bin of
+//               the new cell; writes the next state in the current slot
+//               order to the "n*" buffers.
+//   k_rebuild   bins -> cstart and canonical order (cells ascending, within
+//               a cell ascending previous slot, i.e. a stable counting
+//               sort); positions and ids move into it; the positions the
+//               step started from (pos0 of the next step, re-imaged when
+//               read), the forces and the memory stay where the step had or
+//               wrote them (read through the slot map prev).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -91,49 +86,27 @@ int collect_times(psim_ctx *c)
     return 0;
 }
 
-// counts (already accumulated) -> cstart, scatter, canonical move.
+// The bins (already filled) -> start table, canonical order.
 int launch_build(psim_ctx *c, StepCtl *advance)
 {
-    const int n = c->n, nc = c->ncell;
-    hipStream_t st = c->stream;
-    const bool direct = c->nscan <= kScanDirectTiles;
-    if (direct) {
-        k_scan_direct<<<c->nscan, kScanThreads, 0, st>>>(c->count, nc, c->cstart, n,
-                                                         c->rec.cstart);
-    } else {
-        launch_scan3(st, c->count, nc, c->nscan, c->bsum, c->cstart, n, c->rec.cstart);
-    }
-    if (n >= kMoveIlpMin)
-        k_scatter<kMoveIlp><<<blocks_for(n, 256 * kMoveIlp), 256, 0, st>>>(
-            n, c->key, c->arank, c->cstart, c->perm, direct ? c->count : nullptr, nc);
-    else
-        k_scatter<1><<<blocks_for(n, 256), 256, 0, st>>>(n, c->key, c->arank, c->cstart,
-                                                         c->perm, direct ? c->count : nullptr,
-                                                         nc);
     // positions and ids move into the new order, the positions into the
     // buffer of the last step's start positions (read by this step's
     // integrator, not after it); the positions this step started from become
     // pos0, and they, the forces and the memory stay where this step had or
     // wrote them (old order): the next step reads them through prev
-    auto move = [&](auto box) {
-        if (n >= kMoveIlpMin)
-            k_move_lagged<kMoveIlp><<<blocks_for(n, 256 * kMoveIlp), 256, 0, st>>>(
-                n, c->perm, c->key, c->cstart, c->npos, c->id, c->pos0, c->nid, c->prev, advance,
-                c->upos, box, c->rec.pos, c->rec.id, c->rec.inv);
-        else
-            k_move_lagged<1><<<blocks_for(n, 256), 256, 0, st>>>(
-                n, c->perm, c->key, c->cstart, c->npos, c->id, c->pos0, c->nid, c->prev, advance,
-                c->upos, box, c->rec.pos, c->rec.id, c->rec.inv);
-    };
+    const Rebuilt to{c->cstart, c->pos0, c->nid, c->prev, c->upos,
+                     c->rec.cstart, c->rec.pos, c->rec.id, c->rec.inv};
     if (c->upos)
-        move(OneBox{c->cull.inv_L});
+        launch_rebuild(c->stream, c->n, c->ncell, c->bins, c->npos, c->id, advance,
+                       OneBox{c->cull.inv_L}, to);
     else
-        move(NoBox{});
+        launch_rebuild(c->stream, c->n, c->ncell, c->bins, c->npos, c->id, advance, NoBox{}, to);
     CK(hipGetLastError());
     std::swap(c->id, c->nid);
     std::swap(c->pos, c->pos0);
     std::swap(c->frc, c->nfrc);
     std::swap(c->mem, c->nmem);
+    std::swap(c->bins.b.tile_total, c->bins.next_total);
     c->lagged = true;
     return 0;
 }
@@ -351,8 +324,7 @@ StepArgs step_args(psim_ctx *c, const double *noise, const StepCtl *ctl)
     a.prev = c->lagged ? c->prev : nullptr;
     a.x0_raw = c->lagged ? 1 : 0;
     a.npos = c->npos; a.npos0 = c->npos0; a.nfrc = c->nfrc; a.nmem = c->nmem;
-    a.nid = nullptr; a.vel = c->vel; a.key = c->key; a.arank = c->arank;
-    a.count = c->count; a.err = c->err;
+    a.vel = c->vel; a.bins = c->bins.b; a.err = c->err;
     a.pbc = c->pbc;
     a.noise = noise;
     a.seed = c->prm.seed;
@@ -410,7 +382,7 @@ GraphKey graph_key(const psim_ctx *c)
     GraphKey k{};
     k.pos = c->pos; k.pos0 = c->pos0; k.frc = c->frc; k.mem = c->mem;
     k.npos = c->npos; k.npos0 = c->npos0; k.nfrc = c->nfrc; k.nmem = c->nmem;
-    k.id = c->id; k.nid = c->nid; k.pbc = c->pbc;
+    k.id = c->id; k.nid = c->nid; k.pbc = c->pbc; k.totals = c->bins.b.tile_total;
     k.geo = c->geo; k.pot = c->pot; k.gb = c->gb; k.seed = c->prm.seed;
     return k;
 }
@@ -606,9 +578,8 @@ int set_state(psim_ctx *c, const double *pos, const double *pos0, const double *
     if ((rc = soa(frc, c->nfrc, false, true))) return rc;
     if ((rc = soa(memx, c->nmem, false, true))) return rc;
     CK(hipMemcpyAsync(c->id, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
-    CK(hipMemsetAsync(c->count, 0, sizeof(int) * c->ncell, c->stream));
-    k_hash_count<<<blocks_for(n, 256), 256, 0, c->stream>>>(c->geo, c->npos, c->key,
-                                                            c->arank, c->count);
+    CK(clear_bins(c->stream, n, c->ncell, c->bins));
+    k_bin_all<<<blocks_for(n, 256), 256, 0, c->stream>>>(c->geo, c->npos, c->bins.b);
     CK(hipGetLastError());
     rc = launch_build(c);
     if (rc) return rc;
@@ -679,7 +650,7 @@ int psim_gpu_create(const psim_params *params, psim_ctx **out)
     fill_constants(c);
     c->n = P.n_particles;
     c->ncell = c->geo.ncell;
-    c->nscan = (c->ncell + kScanTile - 1) / kScanTile;
+    shape_bins(c->n, c->ncell, std::pow(c->geo.cell / (2.0 * P.radius), 3.0), c->bins);
     const PathChoice path = choose_path(P, c->geo);
     c->dense = path.dense;
     c->brick = path.brick;
@@ -701,17 +672,12 @@ int psim_gpu_create(const psim_params *params, psim_ctx **out)
     if (!rc && !c->dense && !c->brick) rc = dalloc(&c->upos, c->n);
     if (!rc) rc = dalloc(&c->id, c->n);
     if (!rc) rc = dalloc(&c->nid, c->n);
-    if (!rc) rc = dalloc(&c->key, c->n);
-    if (!rc) rc = dalloc(&c->arank, c->n);
-    if (!rc) rc = dalloc(&c->perm, c->n);
     if (!rc) rc = dalloc(&c->prev, c->n);
     if (!rc) rc = dalloc(&c->ctl, 1);
-    if (!rc) rc = dalloc(&c->count, c->ncell);
+    if (!rc) rc = alloc_bins(c->n, c->ncell, c->bins, [](int **p, size_t k) { return dalloc(p, k); });
     if (!rc) rc = dalloc(&c->cstart, (size_t)c->ncell + 1);
-    if (!rc) rc = dalloc(&c->bsum, (size_t)c->nscan);
     if (!rc) rc = dalloc(&c->err, 1);
-    if (!rc && hipMemsetAsync(c->count, 0, sizeof(int) * c->ncell, c->stream) != hipSuccess)
-        rc = PSIM_E_HIP;
+    if (!rc && clear_bins(c->stream, c->n, c->ncell, c->bins) != hipSuccess) rc = PSIM_E_HIP;
     if (!rc && hipMemsetAsync(c->err, 0, sizeof(DevErr), c->stream) != hipSuccess)
         rc = PSIM_E_HIP;
     // the five arrays of a state, each at an aligned place
@@ -760,8 +726,8 @@ void psim_gpu_destroy(psim_ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
     void *bufs[] = {c->pos, c->pos0, c->frc, c->mem, c->npos, c->npos0, c->nfrc,
-                    c->nmem, c->vel, c->fout, c->upos, c->tupos, c->id, c->nid, c->key, c->arank,
-                    c->perm, c->prev, c->ctl, c->count, c->cstart, c->bsum, c->err, c->noise,
+                    c->nmem, c->vel, c->fout, c->upos, c->tupos, c->id, c->nid,
+                    c->prev, c->ctl, c->cstart, c->err, c->noise,
                     c->tsorted, c->thi, c->tcse, c->st_count, c->st_hash, c->pbc,
                     c->track0, c->hg.key,
                     c->hg.rank, c->hg.perm, c->hg.count, c->hg.cstart, c->hg.bsum,
@@ -769,6 +735,7 @@ void psim_gpu_destroy(psim_ctx *c)
                     c->work, c->iwork};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    free_bins(c->bins);
     stage_free(c->stage);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);

@@ -50,7 +50,7 @@ struct RepGeo {
     BrickGeo bg;   // the replica's bricks (brick kernel)
 };
 
-// 1 / L of the box of slot t (k_move_lagged): rep_of names the replica of
+// 1 / L of the box of slot t (k_rebuild): rep_of names the replica of
 // slots 0, 256, 512, ...; the replica of t is that one or a later one.
 struct ReplicaBox {
     static constexpr bool kPack = true;
@@ -267,16 +267,14 @@ __global__ void k_export_ens(int n, const RepGeo *__restrict__ reps, const int *
 
 // Initial hash of every particle into its replica's cells.
 __global__ void k_ens_hash(const RepGeo *__restrict__ reps, const int *__restrict__ p0,
-                           int nrep, int ntot, const double *pos, const int *id, int *key,
-                           int *arank, int *count)
+                           int nrep, int ntot, const double *pos, const int *id, Bins b)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= ntot) return;
     const Geo g = reps[replica_of(p0, nrep, id[s])].g;
     const int k = g.c0 + cell_1d(pos[s], g.cell, g.S) + g.S * cell_1d(pos[ntot + s], g.cell, g.S)
                 + g.S2 * cell_1d(pos[2 * ntot + s], g.cell, g.S);
-    key[s] = k;
-    arank[s] = wave_aggregated_rank(count, k);
+    bin_particle(b, ntot, s, k);
 }
 
 constexpr int kEnsBlocks[3] = {64, 128, 256};
@@ -305,7 +303,7 @@ struct EnsClass {
 struct psim_ens {
     psim_params common;
     GB gb;
-    int nrep = 0, ntot = 0, ncell = 0, nscan = 0;
+    int nrep = 0, ntot = 0, ncell = 0;
     int mask = 0;
     bool brick = false;  // initial pair kernel of every class: bricks
     int block = 256;     // initial workgroup size / brick target
@@ -328,8 +326,8 @@ struct psim_ens {
     double *vel = nullptr;
     uint4 *upos = nullptr;       // box fractions and cells of pos
     int *rep_of = nullptr;       // replica of slots 0, 256, 512, ...
-    int *id = nullptr, *nid = nullptr, *key = nullptr, *arank = nullptr, *perm = nullptr;
-    int *count = nullptr, *cstart = nullptr, *bsum = nullptr;
+    int *id = nullptr, *nid = nullptr, *cstart = nullptr;
+    BinStore bins;   // members of the cells after the step
     // pos0 / frc / mem stay in the slot order of the last step (pos0: the
     // positions it started from, re-imaged when read); prev[s] is the slot
     // in that order of the particle now in slot s
@@ -382,8 +380,7 @@ StepArgs ens_args(psim_ens *e)
     a.prev = e->lagged ? e->prev : nullptr;
     a.x0_raw = e->lagged ? 1 : 0;
     a.npos = e->npos; a.npos0 = e->npos0; a.nfrc = e->nfrc; a.nmem = e->nmem;
-    a.nid = nullptr; a.vel = e->vel; a.key = e->key; a.arank = e->arank;
-    a.count = e->count; a.err = e->err;
+    a.vel = e->vel; a.bins = e->bins.b; a.err = e->err;
     a.noise = nullptr;
     a.seed = e->common.seed;
     a.ctl = e->ctl;
@@ -436,38 +433,20 @@ void swap_lagged(psim_ens *e)
     std::swap(e->pos, e->pos0);
     std::swap(e->frc, e->nfrc);
     std::swap(e->mem, e->nmem);
+    std::swap(e->bins.b.tile_total, e->bins.next_total);
 }
 
 void launch_build_ens(psim_ens *e, StepCtl *advance)
 {
-    const int n = e->ntot, nc = e->ncell;
-    hipStream_t st = e->stream;
-    const bool direct = e->nscan <= kScanDirectTiles;
-    if (direct) {
-        k_scan_direct<<<e->nscan, kScanThreads, 0, st>>>(e->count, nc, e->cstart, n);
-    } else {
-        launch_scan3(st, e->count, nc, e->nscan, e->bsum, e->cstart, n);
-    }
-    if (n >= kMoveIlpMin)
-        k_scatter<kMoveIlp><<<eblocks(n, 256 * kMoveIlp), 256, 0, st>>>(
-            n, e->key, e->arank, e->cstart, e->perm, direct ? e->count : nullptr, nc);
-    else
-        k_scatter<1><<<eblocks(n, 256), 256, 0, st>>>(n, e->key, e->arank, e->cstart, e->perm,
-                                                      direct ? e->count : nullptr, nc);
     // positions and ids move into the new order, the positions into the
     // buffer of the last step's start positions (read by this step's
     // integrator, not after it); the positions this step started from become
     // pos0, and they, the forces and the memory stay where this step had or
     // wrote them: the next step reads them through prev
-    const ReplicaBox box{e->rep_of, e->p0, e->reps};
-    if (n >= kMoveIlpMin)
-        k_move_lagged<kMoveIlp><<<eblocks(n, 256 * kMoveIlp), 256, 0, st>>>(
-            n, e->perm, e->key, e->cstart, e->npos, e->id, e->pos0, e->nid, e->prev, advance,
-            e->upos, box);
-    else
-        k_move_lagged<1><<<eblocks(n, 256), 256, 0, st>>>(
-            n, e->perm, e->key, e->cstart, e->npos, e->id, e->pos0, e->nid, e->prev, advance,
-            e->upos, box);
+    launch_rebuild(e->stream, e->ntot, e->ncell, e->bins, e->npos, e->id, advance,
+                   ReplicaBox{e->rep_of, e->p0, e->reps},
+                   Rebuilt{e->cstart, e->pos0, e->nid, e->prev, e->upos, nullptr, nullptr,
+                           nullptr, nullptr});
     swap_lagged(e);
     e->lagged = true;
 }
@@ -673,7 +652,10 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
     e->ntot = (int)ntot;
     e->ncell = (int)ncell;
     for (auto &rg : h) rg.g.n = e->ntot;   // SoA stride of the stacked arrays
-    e->nscan = (e->ncell + kScanTile - 1) / kScanTile;
+    double volume = 0.0;
+    for (int r = 0; r < nrep; ++r)
+        volume = std::max(volume, std::pow(h[r].g.cell / (2.0 * e->common.radius), 3.0));
+    shape_bins(e->ntot, e->ncell, volume, e->bins);
     const size_t n3 = 3 * (size_t)e->ntot;
     int rc = 0;
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) rc = PSIM_E_HIP;
@@ -681,7 +663,7 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
                         &e->nmem, &e->vel};
     for (double **b : dbufs)
         if (!rc) rc = ealloc(b, n3);
-    int **ibufs[] = {&e->id, &e->nid, &e->key, &e->arank, &e->perm, &e->prev};
+    int **ibufs[] = {&e->id, &e->nid, &e->prev};
     for (int **b : ibufs)
         if (!rc) rc = ealloc(b, (size_t)e->ntot);
     if (!rc) rc = ealloc(&e->upos, (size_t)e->ntot);
@@ -694,9 +676,9 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
     if (!rc && hipMemcpy(e->rep_of, rep_of.data(), sizeof(int) * rep_of.size(),
                          hipMemcpyHostToDevice) != hipSuccess)
         rc = PSIM_E_HIP;
-    if (!rc) rc = ealloc(&e->count, (size_t)e->ncell);
+    if (!rc)
+        rc = alloc_bins(e->ntot, e->ncell, e->bins, [](int **p, size_t k) { return ealloc(p, k); });
     if (!rc) rc = ealloc(&e->cstart, (size_t)e->ncell + 1);
-    if (!rc) rc = ealloc(&e->bsum, (size_t)e->nscan);
     if (!rc) rc = ealloc(&e->err, 1);
     if (!rc) rc = ealloc(&e->ctl, 1);
     if (!rc) rc = ealloc(&e->reps, (size_t)nrep);
@@ -732,7 +714,7 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
     }
     if (!rc && hipMemcpy(e->p0, e->h_p0.data(), sizeof(int) * (nrep + 1), hipMemcpyHostToDevice) != hipSuccess)
         rc = PSIM_E_HIP;
-    if (!rc && hipMemset(e->count, 0, sizeof(int) * e->ncell) != hipSuccess) rc = PSIM_E_HIP;
+    if (!rc && clear_bins(e->stream, e->ntot, e->ncell, e->bins) != hipSuccess) rc = PSIM_E_HIP;
     if (!rc && hipMemset(e->err, 0, sizeof(DevErr)) != hipSuccess) rc = PSIM_E_HIP;
     // the four arrays of a state, each at an aligned place
     if (!rc && !stage_reserve(e->stage, 4 * (sizeof(double) * n3 + 64))) rc = PSIM_E_HIP;
@@ -750,11 +732,11 @@ void psim_ens_destroy(psim_ens *e)
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     drop_graph(e);
     void *bufs[] = {e->pos, e->pos0, e->frc, e->mem, e->npos, e->npos0, e->nfrc, e->nmem,
-                    e->vel, e->id, e->nid, e->key, e->arank, e->perm, e->count, e->cstart,
-                    e->bsum, e->err, e->ctl, e->reps, e->p0, e->integ_wg, e->st_count,
+                    e->vel, e->id, e->nid, e->cstart, e->err, e->ctl, e->reps, e->p0, e->integ_wg, e->st_count,
                     e->st_hash, e->prev, e->upos, e->rep_of};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    free_bins(e->bins);
     stage_free(e->stage);
     for (EnsClass &cl : e->cls) {   // the occupancy classes and the all-replica one
         void *cb[] = {cl.rmap, cl.wg, cl.item0};
@@ -801,7 +783,7 @@ int psim_ens_set_state(psim_ens *e, const double *pos, const double *vel, double
     std::vector<int> ids(n);
     for (int i = 0; i < n; ++i) ids[i] = i;
     ECK(hipMemcpy(e->id, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-    ECK(hipMemset(e->count, 0, sizeof(int) * e->ncell));
+    ECK(clear_bins(e->stream, e->ntot, e->ncell, e->bins));
     StepCtl c{};
     c.step = 0;
     c.time = current_time;
@@ -817,7 +799,7 @@ int psim_ens_set_state(psim_ens *e, const double *pos, const double *vel, double
     }
     ECK(hipMemcpy(e->ctl, &c, sizeof(c), hipMemcpyHostToDevice));
     k_ens_hash<<<eblocks(n, 256), 256, 0, e->stream>>>(e->reps, e->p0, e->nrep, n, e->npos,
-                                                       e->id, e->key, e->arank, e->count);
+                                                       e->id, e->bins.b);
     launch_build_ens(e, nullptr);
     ECK(hipGetLastError());
     // the fresh previous positions (already re-imaged, upload order), forces

@@ -93,9 +93,8 @@ struct StepArgs {
     int x0_raw;          // pos0 holds the positions the last step started from (re-imaged
                          // here against the current ones); npos0 is then not written
     double *npos, *npos0, *nfrc, *nmem;
-    int *nid;            // copy of id in the current order (null: not kept)
     double *vel;         // [3][N] by original index
-    int *key, *arank, *count;
+    Bins bins;
     DevErr *err;
     const double *noise; // [6][N] by original index, or null -> Philox
     unsigned long long seed, step;
@@ -106,7 +105,7 @@ struct StepArgs {
 
 // G&B epilogue for the particle in slot s with total force F
 // (brownianIntegrator.cpp:191-356, particle.cpp:61-99); writes the next state
-// at slot s, the new cell key and an atomic per-cell rank.
+// at slot s and enters it in its new cell's bin.
 // (o = id[s] and ps = prev[s] may be read by the caller ahead of the force
 // loop, so that their latency overlaps it: pass them as o_pre / ps_pre.)
 template <bool WRITE_F>
@@ -207,12 +206,10 @@ __device__ __forceinline__ void integrate_one(const Geo &g, const GB &gb, const 
         if (WRITE_F) a.nfrc[d * N + s] = F[d];
         a.nmem[d * N + s] = M[d];
     }
-    if (a.nid) a.nid[s] = o;
     if (bad) report_error(a.err, 7703, o, -1);
     int k = g.c0 + cell_1d(xw[0], g.cell, g.S) + g.S * cell_1d(xw[1], g.cell, g.S)
           + g.S2 * cell_1d(xw[2], g.cell, g.S);
-    a.key[s] = k;
-    a.arank[s] = wave_aggregated_rank(a.count, k);
+    bin_particle(a.bins, N, s, k);
 }
 
 // Thread-per-particle step (sparse systems and S < 4); with SPLIT > 1,
