@@ -110,18 +110,14 @@ struct StepArgs {
 // loop, so that their latency overlaps it: pass them as o_pre / ps_pre.)
 template <bool WRITE_F>
 __device__ __forceinline__ void integrate_one(const Geo &g, const GB &gb, const StepArgs &a, int s,
-                              double fx, double fy, double fz, int o_pre = -1, int ps_pre = -1,
-                              const double *z_pre = nullptr)
+                              double fx, double fy, double fz, int o_pre = -1, int ps_pre = -1)
 {
     const int N = g.n;
     const int o = o_pre >= 0 ? o_pre : a.id[s];
     const int first = a.ctl ? a.ctl->first : a.first;
     const int do_vel = a.ctl ? a.ctl->do_vel : a.do_vel;
     double z[6];
-    if (z_pre) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) z[k] = z_pre[k];
-    } else if (a.noise) {
+    if (a.noise) {
 #pragma unroll
         for (int k = 0; k < 6; ++k) z[k] = a.noise[(size_t)k * N + o];
     } else {
@@ -212,6 +208,88 @@ __device__ __forceinline__ void integrate_one(const Geo &g, const GB &gb, const 
     bin_particle(a.bins, N, s, k);
 }
 
+// integrate_one<true> with four consecutive lanes per particle: lane sub =
+// 0..2 makes one Box-Muller pair and takes one dimension, with that component
+// f of the force; lane 3 only takes part in the exchanges.  The operations on
+// a value are integrate_one's, so the results are the same bits.
+// The epilogue is some thousand FP64 instructions, most of them noise; on one
+// lane in four every wave still issues them all.  A step before -> after:
+// 30,011 LJ 26.7 -> 24.5 us, 60,000 AO 19.6 -> 18.1; a fit iteration at 32,768
+// AO 7.05 -> 6.78 ms.  (The separate integrator of the dense path gains
+// nothing from it: it waits for memory.  4,096 LJ+CAL 18.8 -> 18.25, 2,000
+// and 16,500 no difference, a single step of 1,000 0.9 us slower.)
+__device__ __forceinline__ void integrate_quad(const Geo &g, const GB &gb, const StepArgs &a,
+                                               int s, bool valid, int sub, int o, int ps,
+                                               double f)
+{
+    const int N = g.n;
+    const int first = a.ctl ? a.ctl->first : a.first;
+    const int do_vel = a.ctl ? a.ctl->do_vel : a.do_vel;
+    const int d = sub < 3 ? sub : 2;
+    const bool mine = valid && sub < 3;
+    const double xc = a.pos[d * N + s];
+    double x0c = a.pos0[d * N + ps];
+    const double Mo = a.mem[d * N + ps], Fo = a.frc[d * N + ps];
+    double zc, M;   // normals d and 3 + d of the particle
+    if (a.noise) {
+        zc = a.noise[(size_t)d * N + o];
+        M = a.noise[(size_t)(3 + d) * N + o];
+    } else {
+        double za, zb;   // normals 2 sub and 2 sub + 1
+        philox_pair(a.seed, a.ctl ? a.ctl->step : a.step, (uint32_t)o, d, za, zb);
+        const int base = (int)(threadIdx.x & 63u) & ~3;
+        // 0, 1, 2 come from lanes 0, 0, 1; 3, 4, 5 from lanes 1, 2, 2
+        const double ca = __shfl(za, base + (d >> 1), 64), cb = __shfl(zb, base, 64);
+        const double ma = __shfl(za, base + 2, 64), mb = __shfl(zb, base + 1 + (d >> 1), 64);
+        zc = d == 1 ? cb : ca;
+        M = d == 1 ? ma : mb;
+    }
+    if (a.x0_raw) x0c = safe_mod0(x0c, xc, g.L);
+    double xn;
+    if (first) {
+        const double v = a.vel[(size_t)d * N + o];
+        xn = xc + (v * gb.coeff1 * gb.dt) + (f * gb.coeff3 * gb.dt * gb.dt * gb.m) +
+             (gb.sig1 * M);
+    } else {
+        const double Cr = gb.sig2 * ((gb.corr * Mo) + (gb.dev * zc));
+        xn = (gb.c0 * xc);
+        xn -= (gb.coeff0 * x0c);
+        xn += (gb.c1 * f);
+        xn += (gb.c2 * (f - Fo));
+        xn += (gb.sig1 * M) + (gb.coeff0 * Cr);
+        if (do_vel) {
+            const double xN = safe_mod(xn, g.L);
+            const double dx = xN - safe_mod0(xc, xN, g.L);
+            double vv = dx + (xc - x0c);
+            vv += (gb.g2 * f);
+            vv -= (gb.g3 * (f - Fo));
+            vv += (Cr - gb.sig1 * M);
+            vv *= gb.g4;
+            if (mine) a.vel[(size_t)d * N + o] = vv;
+        }
+    }
+    const double xw = safe_mod(xn, g.L);
+    const double x0n = safe_mod0(xc, xw, g.L);
+    int k = cell_1d(xw, g.cell, g.S) * (d == 0 ? 1 : d == 1 ? g.S : g.S2);
+    k = sub < 3 ? k : g.c0;
+    k += __shfl_xor(k, 1, 64);
+    k += __shfl_xor(k, 2, 64);
+    if (mine) {
+        if (a.pbc) {
+            if (x0n < 0)
+                a.pbc[(size_t)d * N + o] += 1;
+            else if (x0n > g.L)
+                a.pbc[(size_t)d * N + o] -= 1;
+        }
+        a.npos[d * N + s] = xw;
+        if (!a.x0_raw) a.npos0[d * N + s] = x0n;
+        a.nfrc[d * N + s] = f;
+        a.nmem[d * N + s] = M;
+        if ((xw < 0.0) || (xw >= g.L)) report_error(a.err, 7703, o, -1);
+    }
+    if (valid && sub == 0) bin_particle(a.bins, N, s, k);
+}
+
 // Thread-per-particle step (sparse systems and S < 4); with SPLIT > 1,
 // SPLIT lanes per particle share its 27 neighbour cells (small systems,
 // where one lane per particle leaves most SIMDs idle and each lane waits
@@ -220,7 +298,7 @@ template <int MASK, int BLOCK, int SPLIT = 1>
 __global__ __launch_bounds__(BLOCK) void k_step(Geo g, Pot p, Cull q, GB gb,
                                                 double radius, StepArgs a)
 {
-    static_assert(SPLIT >= 1 && 64 % SPLIT == 0 && (SPLIT & (SPLIT - 1)) == 0, "lane groups");
+    static_assert(SPLIT == 1 || SPLIT == 4, "lane groups");
     __shared__ WaveLists lists[BLOCK / 64];
     const int t = xcd_block() * BLOCK + threadIdx.x;
     const int sub = t % SPLIT;
@@ -235,32 +313,12 @@ __global__ __launch_bounds__(BLOCK) void k_step(Geo g, Pot p, Cull q, GB gb,
     wave_gather<MASK, SPLIT>(g, p, q, SoAPos{a.pos, N, radius}, StartTab{a.cstart}, a.upos, valid,
                              s, lists[threadIdx.x >> 6], fx, fy, fz, a.err, Orig{a.id, 1, 0},
                              sub);
-    // (not with LJ: its pair arithmetic leaves no registers for the pairs)
-    if constexpr (SPLIT >= 4 && !(MASK & F_LJ)) {
+    if constexpr (SPLIT == 4) {
         fx = split_sum<SPLIT>(fx);
         fy = split_sum<SPLIT>(fy);
         fz = split_sum<SPLIT>(fz);
-        if (!a.noise) {
-            // in-kernel noise: lanes 0..2 of the group each make one
-            // Box-Muller pair, gathered on lane 0
-            double za = 0.0, zb = 0.0;
-            if (sub < 3)
-                philox_pair(a.seed, a.ctl ? a.ctl->step : a.step, (uint32_t)o, sub, za, zb);
-            const int base = (int)(threadIdx.x & 63u) & ~(SPLIT - 1);
-            double z[6];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                z[2 * k] = __shfl(za, base + k, 64);
-                z[2 * k + 1] = __shfl(zb, base + k, 64);
-            }
-            if (sub != 0 || !valid) return;
-            integrate_one<true>(g, gb, a, s, fx, fy, fz, o, ps, z);
-            return;
-        }
-    } else if constexpr (SPLIT > 1) {
-        fx = split_sum<SPLIT>(fx);
-        fy = split_sum<SPLIT>(fy);
-        fz = split_sum<SPLIT>(fz);
+        integrate_quad(g, gb, a, s, valid, sub, o, ps, sub == 0 ? fx : sub == 1 ? fy : fz);
+        return;
     }
     if (sub != 0 || !valid) return;
     integrate_one<true>(g, gb, a, s, fx, fy, fz, o, ps);
