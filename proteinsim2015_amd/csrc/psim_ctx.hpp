@@ -33,6 +33,7 @@ struct psim_ctx {
     psim::Cull cull;   // derived from geo and pot
     int n = 0, ncell = 0;
     bool dense = false;   // cell-per-workgroup pair kernel (else thread per particle)
+    bool cells = false;   // dense: a wave per cell instead of a workgroup
     bool brick = false;   // brick-per-workgroup pair kernel (sparse systems)
     psim::BrickGeo bg{};  // its bricks
     int brick_g = 1;      // its lanes per particle

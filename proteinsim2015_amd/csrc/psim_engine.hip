@@ -195,7 +195,13 @@ void with_lj_exponent(int lj_num, Launch launch)
 template <int MASK>
 void launch_step_mask(psim_ctx *c, const StepArgs &a)
 {
-    if (c->dense) {
+    if (c->cells) {
+        const int per = cells_per_xcd(c->ncell);
+        with_lj_exponent<MASK>(c->pot.lj_num, [&](auto ljn) {
+            k_step_cells<MASK, decltype(ljn)::value><<<8 * per, kCellBlock, 0, c->stream>>>(
+                c->geo, c->pot, c->prm.radius, a.pos, a.id, a.cstart, a.nfrc, a.err, per);
+        });
+    } else if (c->dense) {
         const int per = (c->ncell + 7) / 8;
         with_lj_exponent<MASK>(c->pot.lj_num, [&](auto ljn) {
             k_step_dense<MASK, decltype(ljn)::value><<<8 * per, kDenseThreads, 0, c->stream>>>(
@@ -240,7 +246,13 @@ int launch_step(psim_ctx *c, const StepArgs &a)
 template <int MASK>
 void launch_forces_mask(psim_ctx *c)
 {
-    if (c->dense) {
+    if (c->cells) {
+        const int per = cells_per_xcd(c->ncell);
+        with_lj_exponent<MASK>(c->pot.lj_num, [&](auto ljn) {
+            k_forces_cells<MASK, decltype(ljn)::value><<<8 * per, kCellBlock, 0, c->stream>>>(
+                c->geo, c->pot, c->prm.radius, c->pos, c->id, c->cstart, c->fout, c->err, per);
+        });
+    } else if (c->dense) {
         const int per = (c->ncell + 7) / 8;
         with_lj_exponent<MASK>(c->pot.lj_num, [&](auto ljn) {
             k_forces_dense<MASK, decltype(ljn)::value>
@@ -653,6 +665,7 @@ int psim_gpu_create(const psim_params *params, psim_ctx **out)
     shape_bins(c->n, c->ncell, std::pow(c->geo.cell / (2.0 * P.radius), 3.0), c->bins);
     const PathChoice path = choose_path(P, c->geo);
     c->dense = path.dense;
+    c->cells = path.cells;
     c->brick = path.brick;
     c->brick_g = path.brick_g;
     c->bg = path.bg;

@@ -135,8 +135,14 @@ void launch_forces_aos(const psim_params &P, const Geo &geo, const Pot &pot, con
 {
     const int n = geo.n;
     if (path.dense) {
-        const int per = (geo.ncell + 7) / 8;
+        const int per = path.cells ? cells_per_xcd(geo.ncell) : (geo.ncell + 7) / 8;
         auto launch = [&](auto ljn) {
+            if (path.cells) {
+                k_forces_cells<MASK, decltype(ljn)::value>
+                    <<<8 * per, kCellBlock, 0, st>>>(geo, pot, P.radius, pos, id, cstart, fout,
+                                                     err, per);
+                return;
+            }
             k_forces_dense<MASK, decltype(ljn)::value>
                 <<<8 * per, kDenseThreads, 0, st>>>(geo, pot, P.radius, pos, id, cstart, fout,
                                                     err, per);

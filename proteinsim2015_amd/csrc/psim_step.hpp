@@ -6,6 +6,7 @@
 #include <cmath>
 
 #include "psim_brick.hpp"
+#include "psim_cells.hpp"
 #include "psim_dense.hpp"
 #include "psim_gather.hpp"
 #include "psim_gpu.h"
@@ -15,20 +16,17 @@
 namespace psim {
 namespace {
 
-// Mean particles per cell from which the cell-per-workgroup kernel beats the
-// thread-per-particle one.  The former's time grows with the cells (a
-// workgroup each, of which the chip holds 1792 at once), the latter's with the
-// candidates per particle, at four lanes per particle below kSmallSystem and
-// one above.  Measured on MI355X, whole steps (thread per particle / cell per
-// workgroup, us): N = 4096 at 2.4 per cell 21 / 24, at 3.1 26 / 24; 16,384 at
-// 4.0 33 / 35, at 4.9 36 / 31; 32,768 at 3.1 33 / 52, at 6.7 45 / 36; 65,536 at
-// 5.4 55 / 59, at 6.2 59 / 55; 262,144 at 6.1 117 / 151, at 8.0 149 / 143;
-// 1,048,576 at 3.1 249 / 1016, at 7.9 518 / 510, at 9.5 566 / 425.
-inline double dense_min_occupancy(int n)
-{
-    if (n >= 256 * 1024) return 8.0;
-    return std::min(5.7, std::max(2.7, 2.7 + std::log2(n / 6144.0)));
-}
+// Mean particles per cell from which the cell kernels are used.
+constexpr double kDenseMinOccupancy = 2.0;
+// Below this many particles per cell a wave takes a cell instead of a
+// workgroup, in systems of this size: a workgroup's time is mostly the same
+// for every cell, a wave's grows with the cell's pairs and is the longer one
+// where there are too few cells to fill the chip.  Whole steps (workgroup /
+// wave, us) at 2.2 per cell: N = 30,011 54 / 38, 200,000 277 / 141; at 3.0:
+// 10,000 26.1 / 26.9, 16,000 32.4 / 28.6, 30,011 45 / 38, 200,000 210 / 137;
+// at 3.9: 30,011 38 / 45, 60,000 58 / 59; at 4.8: 200,000 139 / 183.
+constexpr double kCellsMaxOccupancy = 3.5;
+constexpr int kCellsMin = 12288;
 // below this many particles the thread-per-particle kernels use 64-lane
 // blocks (256-lane blocks would leave CUs idle: 256 CUs x 4 blocks)
 constexpr int kSmallSystem = 256 * 1024;
@@ -57,13 +55,14 @@ inline int check_params(const psim_params &P)
     return 0;
 }
 
-// Pair-kernel path of a system: the cell-per-workgroup kernel needs S >= 4
-// (shifted image = minimum image) and pays off once cells hold a few
-// particles (dense_min_occupancy); below that, one thread per particle (bricks of cells per
+// Pair-kernel path of a system: the cell kernels need S >= 4 (shifted image =
+// minimum image) and pay off once cells hold a few particles, a wave per cell
+// first, then a workgroup; below that, one thread per particle (bricks of cells per
 // workgroup, path 3, give the same bits but measured slower at every sparse
 // density).
 struct PathChoice {
     bool dense;
+    bool cells;    // a wave per cell instead of a workgroup (the same bits)
     bool brick;
     int brick_g;   // lanes per particle of the brick step kernel
     BrickGeo bg;
@@ -77,7 +76,8 @@ inline PathChoice choose_path(const psim_params &P, const Geo &g)
     else if (P.kernel_path == 2)
         c.dense = g.S >= 4;
     else
-        c.dense = g.S >= 4 && occupancy >= dense_min_occupancy(g.n);
+        c.dense = g.S >= 4 && occupancy >= kDenseMinOccupancy;
+    c.cells = c.dense && occupancy < kCellsMaxOccupancy && g.n >= kCellsMin;
     c.brick = P.kernel_path == 3;
     c.brick_g = g.n < kSmallSystem ? kSmallSplit : 1;
     c.bg = brick_shape(g.S, occupancy, kBrickTarget * kBrickThreads / c.brick_g);
@@ -367,6 +367,23 @@ __attribute__((amdgpu_waves_per_eu(dense_waves(MASK, LJN)))) void k_step_dense(
                             });
 }
 
+// Wave-per-cell forces for the step (the same bits as k_step_dense).
+template <int MASK, int LJN>
+__global__ __launch_bounds__(kCellBlock)
+__attribute__((amdgpu_waves_per_eu(cell_waves(MASK)))) void k_step_cells(Geo g, Pot p, double radius,
+                                                           const double *pos, const int *id,
+                                                           const int *cstart, double *nfrc,
+                                                           DevErr *err, int per_xcd)
+{
+    const int N = g.n;
+    cells_forces<MASK, LJN>(g, p, radius, pos, cstart, id, err, per_xcd,
+                            [=](int s, double Fx, double Fy, double Fz) {
+                                nfrc[s] = Fx;
+                                nfrc[N + s] = Fy;
+                                nfrc[2 * N + s] = Fz;
+                            });
+}
+
 // G&B step for every slot with the force already in nfrc (dense path).
 __global__ __launch_bounds__(256) void k_integrate(Geo g, GB gb, StepArgs a)
 {
@@ -435,6 +452,27 @@ __attribute__((amdgpu_waves_per_eu(dense_waves(MASK, LJN)))) void k_forces_dense
                             [=](int i, double Fx, double Fy, double Fz) {
                                 store_aos(fout, id[home0 + i], Fx, Fy, Fz);
                             });
+}
+
+// Forces only, wave per cell (the same bits as k_forces_dense).
+template <int MASK, int LJN>
+__global__ __launch_bounds__(kCellBlock)
+__attribute__((amdgpu_waves_per_eu(cell_waves(MASK)))) void k_forces_cells(Geo g, Pot p, double radius,
+                                                             const double *pos, const int *id,
+                                                             const int *cstart, double *fout,
+                                                             DevErr *err, int per_xcd)
+{
+    cells_forces<MASK, LJN>(g, p, radius, pos, cstart, id, err, per_xcd,
+                            [=](int s, double Fx, double Fy, double Fz) {
+                                store_aos(fout, id[s], Fx, Fy, Fz);
+                            });
+}
+
+// Grid of the wave-per-cell kernels and its per_xcd.
+inline int cells_per_xcd(int ncell)
+{
+    constexpr int kWaves = kCellBlock / 64;
+    return ((ncell + kWaves - 1) / kWaves + 7) / 8;
 }
 
 // ---------------------------------------------------------------------------
