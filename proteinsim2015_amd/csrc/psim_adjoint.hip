@@ -47,7 +47,7 @@ using eng::dalloc;
 namespace {
 
 constexpr int kAdjBlock = 256;
-constexpr int kAdjSmall = 256 * 1024;   // below this N, 8 lanes per particle
+constexpr int kAdjSmall = 256 * 1024;   // below this N, 8 lanes per particle, else 2
 constexpr int kNTheta = 5;   // AO wellDepth, AO cutOff, LJ wellDepth, yukawaStrength, debyeLength
 
 // Host-side derivatives of the pair constants (AOPotential.cpp:50-55).
@@ -128,11 +128,11 @@ __device__ __forceinline__ void pair_fnet_d(const Pot &p, const AdjPot &q, doubl
 }
 
 // Pairs of slot s inside the cutoff, with the forward kernels' neighbour
-// test and displacement (psim_pairs.hpp gather_force / drain_hits), as
+// test and displacement (psim_gather.hpp), as
 // fn(j, dx, dy, dz, r, 1/r, true); with win_hi2 > 0 also the pairs outside
 // it with r^2 < win_hi2, as fn(..., false).  Lane `sub` of the SPLIT lanes
 // that share the particle visits the x-runs sub, sub + SPLIT, ... of the 9
-// (gather_force's walk).
+// (the forward kernels' rows).
 template <bool EXACT, int SPLIT, class Fn>
 __device__ void visit_pairs(const Geo &g, const Pot &p, const double *pos, const int *cstart,
                             int s, int sub, double win_hi2, Fn fn)
@@ -190,6 +190,10 @@ __device__ void visit_pairs(const Geo &g, const Pot &p, const double *pos, const
 // is read at its slot; lambda_{n-1} goes to lam_prev in the slot order of
 // the state before (inv: original index -> slot there) or, with inv null, by
 // original index.  The a_n are kept by original index.
+// Bound by the latency of its chain of loads (cell table, candidates, their
+// lambda); what the end of the step reads is loaded ahead of the pairs.
+// (Collecting the pairs and evaluating them 64 at a time, one per lane, took
+// as long: 6.94 ms for 6.80 and 3.89 for 3.95 at the sizes of adj_split.)
 template <int MASK, bool EXACT, int BLOCK, int SPLIT>
 __global__ __launch_bounds__(BLOCK) void k_adj_step(
     Geo g, Pot p, AdjPot q, double radius, const double *pos, const int *id,
@@ -202,6 +206,12 @@ __global__ __launch_bounds__(BLOCK) void k_adj_step(
     const int N = g.n;
     double th[kNTheta] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double jx = 0.0, jy = 0.0, jz = 0.0;
+    // what the end of the step needs, in flight during the pairs: with a group
+    // of lanes each of the first three takes a dimension
+    const int sl = s < N ? s : N - 1;
+    const int o = id[sl], ds = SPLIT >= 4 && sub < 3 ? sub : 0;
+    const int wo = lam_prev && inv ? inv[o] : o;
+    const double a1o = a1[(size_t)ds * N + o], a2o = a2[(size_t)ds * N + o];
     if (s < N) {   // whole lane groups
         const double lx = lam[s], ly = lam[N + s], lz = lam[2 * N + s];
         const double size = 2.0 * radius;
@@ -231,19 +241,24 @@ __global__ __launch_bounds__(BLOCK) void k_adj_step(
             jz += __shfl_xor(jz, d, 64);
         }
     }
-    if (s < N && sub == 0) {
-        const int o = id[s];
-        const double n0x = beta * a1[o] - coeff0 * a2[o] + jx;
-        const double n0y = beta * a1[N + o] - coeff0 * a2[N + o] + jy;
-        const double n0z = beta * a1[2 * N + o] - coeff0 * a2[2 * N + o] + jz;
+    if constexpr (SPLIT >= 4) {
+        if (s < N && sub < 3) {
+            const double n0 = beta * a1o - coeff0 * a2o + (sub == 0 ? jx : sub == 1 ? jy : jz);
+            a0[(size_t)ds * N + o] = n0;
+            if (lam_prev) lam_prev[(size_t)ds * N + wo] = alpha_prev * n0 - c2 * a1o;
+        }
+    } else if (s < N && sub == 0) {
+        const double a1y = a1[N + o], a1z = a1[2 * N + o];
+        const double n0x = beta * a1o - coeff0 * a2o + jx;
+        const double n0y = beta * a1y - coeff0 * a2[N + o] + jy;
+        const double n0z = beta * a1z - coeff0 * a2[2 * N + o] + jz;
         a0[o] = n0x;
         a0[N + o] = n0y;
         a0[2 * N + o] = n0z;
         if (lam_prev) {
-            const int w = inv ? inv[o] : o;
-            lam_prev[w] = alpha_prev * n0x - c2 * a1[o];
-            lam_prev[N + w] = alpha_prev * n0y - c2 * a1[N + o];
-            lam_prev[2 * N + w] = alpha_prev * n0z - c2 * a1[2 * N + o];
+            lam_prev[wo] = alpha_prev * n0x - c2 * a1o;
+            lam_prev[N + wo] = alpha_prev * n0y - c2 * a1y;
+            lam_prev[2 * N + wo] = alpha_prev * n0z - c2 * a1z;
         }
     }
     __shared__ double red[kNTheta][BLOCK / 64];
@@ -521,12 +536,15 @@ bool same_forces(const psim_params &a, const psim_params &b)
 }
 
 int adj_block(const psim_ctx *) { return kAdjBlock; }
-// lanes per particle: small systems spread each particle's 27 cells over 8
+// Lanes per particle: small systems spread each particle's 27 cells over 8
 // lanes, so that every CU gets work and each lane waits on fewer lookups
+// (200 steps of 32,768: 8 lanes 6.69 ms, 4 6.92, 16 7.59); larger ones over 2
+// (20 steps of 300,007: one lane 3.92 ms, two 3.73, four 3.95, eight 4.23).
 #ifndef PSIM_ADJ_SPLIT
 #define PSIM_ADJ_SPLIT 8
 #endif
-int adj_split(const psim_ctx *c) { return c->n < kAdjSmall ? PSIM_ADJ_SPLIT : 1; }
+constexpr int kAdjLarge = 2;
+int adj_split(const psim_ctx *c) { return c->n < kAdjSmall ? PSIM_ADJ_SPLIT : kAdjLarge; }
 unsigned adj_blocks(const psim_ctx *c)
 {
     return xcd_grid(blocks_for((long long)c->n * adj_split(c), adj_block(c)));
@@ -567,13 +585,13 @@ void launch_adj_mask(psim_adjoint *A, const AdjPot &q, const double *pos, const 
     k_adj_step<MASK, EX, BL, SP><<<nb, BL, 0, c->stream>>>(                                \
         c->geo, c->pot, q, c->prm.radius, pos, id, cs, lam, a1, a2, a0, lam_prev, inv,     \
         beta, c->gb.coeff0, alpha_prev, c->gb.c2, tp)
-    const bool split = adj_split(c) > 1;
+    const bool split = c->n < kAdjSmall;
     if (c->geo.exact_mi) {
         if (split) PSIM_ADJ_LAUNCH(true, kAdjBlock, PSIM_ADJ_SPLIT);
-        else PSIM_ADJ_LAUNCH(true, kAdjBlock, 1);
+        else PSIM_ADJ_LAUNCH(true, kAdjBlock, kAdjLarge);
     } else {
         if (split) PSIM_ADJ_LAUNCH(false, kAdjBlock, PSIM_ADJ_SPLIT);
-        else PSIM_ADJ_LAUNCH(false, kAdjBlock, 1);
+        else PSIM_ADJ_LAUNCH(false, kAdjBlock, kAdjLarge);
     }
 #undef PSIM_ADJ_LAUNCH
 }
@@ -586,16 +604,16 @@ namespace eng {
 void launch_adj_stats(psim_ctx *c, NbrStatsOut so)
 {
     const unsigned nb = adj_blocks(c);
-    const bool split = adj_split(c) > 1;
+    const bool split = c->n < kAdjSmall;
 #define PSIM_ADJ_STATS(EX, SP)                                                             \
     k_adj_stats<EX, kAdjBlock, SP><<<nb, kAdjBlock, 0, c->stream>>>(c->geo, c->pot, c->pos, \
                                                                     c->id, c->cstart, so)
     if (c->geo.exact_mi) {
         if (split) PSIM_ADJ_STATS(true, PSIM_ADJ_SPLIT);
-        else PSIM_ADJ_STATS(true, 1);
+        else PSIM_ADJ_STATS(true, kAdjLarge);
     } else {
         if (split) PSIM_ADJ_STATS(false, PSIM_ADJ_SPLIT);
-        else PSIM_ADJ_STATS(false, 1);
+        else PSIM_ADJ_STATS(false, kAdjLarge);
     }
 #undef PSIM_ADJ_STATS
 }

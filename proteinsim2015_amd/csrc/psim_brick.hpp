@@ -10,7 +10,7 @@
 // order (x fastest), each load independent of the others.  Then G
 // consecutive lanes take one home particle and run the thread-per-particle
 // gather against LDS: lane gg walks the particle's x-runs gg, gg + G, ...
-// (the 27 neighbour cells of LJPotential.cpp:154-177 in gather_force's
+// (the 27 neighbour cells of LJPotential.cpp:154-177 in the gather's
 // order: (dy, dz) y outer, then dx = -1, 0, +1), candidates in slot order, with
 // k_step's arithmetic (shifted home position per neighbour cell, guard-banded
 // r^2, util::pbcDist's recheck, pair_fr), survivors through a per-lane LDS
@@ -70,7 +70,7 @@ __device__ inline int brick_scan(int v, int *total, int *wsum)
     return before + x - v;
 }
 
-// Pair forces of one lane's hit list, entries [0, nh) (drain_hits' arithmetic
+// Pair forces of one lane's hit list, entries [0, nh) (eval_pair's arithmetic
 // on staged operands).
 template <int MASK, bool EXACT, class ST>
 __device__ __forceinline__ void brick_drain(const Geo &g, const Pot &p, const BrickShared &sh,
