@@ -42,6 +42,11 @@
 // every survivor near or beyond the cutoff is re-tested with util::pbcDist's
 // own arithmetic (utilities.cpp:79-104) against the strict r^2 < rc^2 of
 // LJPotential.cpp:82.
+//
+// Fractions and the nearest image stand for the walk over the cells only where
+// both positions lie in the box.  A pair with one that does not (or is NaN or
+// infinite) takes the image that the walk meets it in (walk_image), so that
+// it is accepted and evaluated as in the kernels that move positions by cell.
 #pragma once
 
 #include "psim_pairs.hpp"
@@ -54,12 +59,50 @@ __device__ __forceinline__ unsigned box_fraction(double x, double inv_L)
     return (unsigned)(__builtin_amdgcn_fract(x * inv_L) * 4294967296.0);
 }
 
-// The cull's copy of a particle: box fractions and the (global) cell index.
+// The cull's copy of a particle: box fractions and the (global) cell index,
+// below 2^31.  Bit 31 of the cell: so many boxes away (or not finite) that the
+// fractions, of 53 bits less those of the number of boxes, are no bound.
+constexpr unsigned kFarAway = 0x80000000u;
 __device__ __forceinline__ uint4 pack_position(double x, double y, double z, int cell,
                                                double inv_L)
 {
+    const bool near = fabs(x * inv_L) + fabs(y * inv_L) + fabs(z * inv_L) < 65536.0;
     return make_uint4(box_fraction(x, inv_L), box_fraction(y, inv_L), box_fraction(z, inv_L),
-                      (unsigned)cell);
+                      (unsigned)cell | (near ? 0u : kFarAway));
+}
+
+// True for every position that is not in [0, L)^3, with a NaN or an infinity
+// too; also for a few that are (-0.0, and x with the high word of L).
+__device__ __forceinline__ unsigned high_word(double x) { return (unsigned)__double2hiint(x); }
+__device__ __forceinline__ bool maybe_outside(double xi, double yi, double zi, double xj,
+                                              double yj, double zj, double L)
+{
+    return max(max(max(high_word(xi), high_word(yi)), high_word(zi)),
+               max(max(high_word(xj), high_word(yj)), high_word(zj))) >= high_word(L);
+}
+
+// The particle at (x, y, z), moved to the image in which the walk over its 27
+// cells meets slot j.
+template <class Tab>
+__device__ inline void walk_image(const Geo &g, const Tab &tab, int j, double &x, double &y,
+                                  double &z)
+{
+    const int S = g.S;
+    const int cx = cell_1d(x, g.cell, S), cy = cell_1d(y, g.cell, S), cz = cell_1d(z, g.cell, S);
+#pragma unroll 1
+    for (int m = 0; m < 9; ++m) {
+        int ry = cy + m / 3 - 1, rz = cz + m % 3 - 1, ky = 0, kz = 0;
+        if (ry < 0) { ry += S; ky = 1; } else if (ry >= S) { ry -= S; ky = 2; }
+        if (rz < 0) { rz += S; kz = 1; } else if (rz >= S) { rz -= S; kz = 2; }
+        const XRun r = x_run(tab, g.c0 + S * ry + g.S2 * rz, cx, S);
+        const bool first = j >= r.b0 && j < r.e0;
+        if (first || (j >= r.b1 && j < r.e1)) {
+            x = shifted(x, first ? r.k0 : r.k1, g.L);
+            y = shifted(y, ky, g.L);
+            z = shifted(z, kz, g.L);
+            return;
+        }
+    }
 }
 
 // upos[j] by a 32-bit byte offset (16 bytes x 2^26 slots)
@@ -113,29 +156,37 @@ __device__ __forceinline__ int wave_inclusive_sum(int x)
 
 // One pair of the evaluation stage: fNet / r of particle j on particle i and
 // the displacement (FP64 positions), or with statistics the acceptance (fr)
-// and the partner's hash (dx).
-template <int MASK, class ST, class Orig_>
-__device__ __forceinline__ void eval_pair(const Geo &g, const Pot &p, const Cull &q, double xi,
+// and the partner's hash (dx).  All are 0 for a pair that is not accepted.
+template <int MASK, class ST, class Tab, class Orig_>
+__device__ __forceinline__ void eval_pair(const Geo &g, const Pot &p, const Cull &q,
+                                          const Tab &tab, double xi,
                                           double yi, double zi, double xj, double yj, double zj,
                                           double size, int si, int j, DevErr *err,
                                           const Orig_ &orig, double &fr, double &dx, double &dy,
                                           double &dz)
 {
-    fr = 0.0;
-    dx = xj - xi;
-    dy = yj - yi;
-    dz = zj - zi;
+    fr = dx = dy = dz = 0.0;
+    double ex = xj - xi, ey = yj - yi, ez = zj - zi;
     double r2, r, rinv;
     if (!g.exact_mi) {
         // the home position moved to the partner's image (by 0 or +-L, exact
         // product), then the difference
-        dx = xj - fma(rint(dx * q.inv_L), g.L, xi);
-        dy = yj - fma(rint(dy * q.inv_L), g.L, yi);
-        dz = zj - fma(rint(dz * q.inv_L), g.L, zi);
-        r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-        if (r2 >= p.rc2_lo) {
+        double hx = fma(rint(ex * q.inv_L), g.L, xi), hy = fma(rint(ey * q.inv_L), g.L, yi),
+               hz = fma(rint(ez * q.inv_L), g.L, zi);
+        // (this test is 1 % of a step at 262,144 AO particles, 32.0 -> 32.4 us)
+        if (maybe_outside(xi, yi, zi, xj, yj, zj, g.L)) {
+            hx = xi;
+            hy = yi;
+            hz = zi;
+            walk_image(g, tab, j, hx, hy, hz);
+        }
+        ex = xj - hx;
+        ey = yj - hy;
+        ez = zj - hz;
+        r2 = fma(ex, ex, fma(ey, ey, ez * ez));
+        if (!(r2 < p.rc2_lo)) {
             const double r2x = pbc_dist_ref(xi, yi, zi, xj, yj, zj, g.L, g.half_pbc);
-            if (!(r2x < p.rc2)) return;
+            if (!(r2 < p.rc2_hi && r2x < p.rc2)) return;
         }
         rinv = rsqrt_nr(r2);
         r = r2 * rinv;
@@ -145,9 +196,9 @@ __device__ __forceinline__ void eval_pair(const Geo &g, const Pot &p, const Cull
         if (!(r2 < p.rc2)) return;
         r = sqrt(r2);
         rinv = 1.0 / r;
-        dx = min_image_uv(dx, g.L, g.half_uv);
-        dy = min_image_uv(dy, g.L, g.half_uv);
-        dz = min_image_uv(dz, g.L, g.half_uv);
+        ex = min_image_uv(ex, g.L, g.half_uv);
+        ey = min_image_uv(ey, g.L, g.half_uv);
+        ez = min_image_uv(ez, g.L, g.half_uv);
     }
     if constexpr (ST::kOn) {
         fr = 1.0;
@@ -161,6 +212,9 @@ __device__ __forceinline__ void eval_pair(const Geo &g, const Pot &p, const Cull
     }
     bool nan_ao = false;
     fr = pair_fr<MASK>(p, rinv, r, size, &nan_ao);
+    dx = ex;
+    dy = ey;
+    dz = ez;
     if (nan_ao) report_error(err, 7705, orig(si), orig(j));
 }
 
@@ -186,11 +240,14 @@ __device__ __forceinline__ void wave_gather(const Geo &g, const Pot &p, const Cu
     // cell coordinates from the cell index: (c + 1/2) / S^2 is at least
     // 1 / (2 S^2) away from a whole number, far above the rounding of the
     // product (S <= 1290)
-    const int c = (int)u.w - g.c0;
+    const int c = (int)(u.w & ~kFarAway) - g.c0;
     const int cz = (int)(((double)c + 0.5) * q.inv_S2);
     const int cyx = c - __mul24(cz, g.S2);
     const int cy = (int)(((float)cyx + 0.5f) * q.inv_S);
     const int cx = cyx - __mul24(cy, S);
+    // (a particle too far away for the cull takes every candidate; one in the
+    // box and one that far away are no pair)
+    const float ucut2 = u.w & kFarAway ? INFINITY : q.ucut2;
     unsigned *col = w.list + lane;
 
     // The cells x-1, x, x+1 of a row as two segments [a0, a1) and [0, b1) of
@@ -270,7 +327,7 @@ __device__ __forceinline__ void wave_gather(const Geo &g, const Pot &p, const Cu
                 const float dx = (float)(int)(v[t].x - u.x), dy = (float)(int)(v[t].y - u.y),
                             dz = (float)(int)(v[t].z - u.z);
                 const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                const bool hit = r2 < q.ucut2 && e[t] != (unsigned)s;
+                const bool hit = r2 < ucut2 && e[t] != (unsigned)s;
                 col[nh * 64] = e[t];   // rows up to k + t have been read
                 nh += hit ? 1 : 0;
             }
@@ -296,7 +353,7 @@ __device__ __forceinline__ void wave_gather(const Geo &g, const Pot &p, const Cu
                 const int si = s0 + i / SPLIT;
                 if (act) {
                     double fr, dx, dy, dz;
-                    eval_pair<MASK, ST>(g, p, q, src.x(si), src.y(si), src.z(si), src.x(j),
+                    eval_pair<MASK, ST>(g, p, q, tab, src.x(si), src.y(si), src.z(si), src.x(j),
                                         src.y(j), src.z(j), src.rad(si) + src.rad(j), si, j, err,
                                         orig, fr, dx, dy, dz);
                     w.pair[t].fr = fr;
