@@ -174,7 +174,11 @@ int psim_gpu_forces(psim_ctx *ctx, double *force_out);
  * (x,y,z,r per sorted index), hash_index = particleHashIndex as 2n ints
  * (hash, original index), cell_start_end = cellStartEnd as 2*S^3 ints
  * (start, end; -1 empty).  force_out is particleForce (AoS3, original
- * index).  n must equal the context's n_particles. */
+ * index).  n must equal the context's n_particles.  The cells must be stored
+ * in cell order along x (as the reference's sort by hash leaves them): the
+ * neighbours x-1, x, x+1 of a row are read from the first non-empty cell's
+ * start to the last one's end, so pairs are missed or met twice in a table
+ * where they are not. */
 int psim_gpu_force_table(psim_ctx *ctx, const double *sorted4,
                          const int *hash_index, const int *cell_start_end,
                          double *force_out);

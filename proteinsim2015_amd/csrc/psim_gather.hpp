@@ -290,7 +290,8 @@ __device__ __forceinline__ void wave_gather(const Geo &g, const Pot &p, const Cu
             for (int sg = 0; sg < 2; ++sg) {
                 int &b = sg ? cur[k].b1 : cur[k].b0;
                 const int e = sg ? cur[k].e1 : cur[k].e0;
-                const int take = min(e - b, kListRows - n), to = b + take;
+                // (a host's table with cells out of row order: b past e)
+                const int take = max(0, min(e - b, kListRows - n)), to = b + take;
                 // two entries at a time (an odd last one spills into the
                 // next free row)
                 unsigned *at = col + n * 64;
