@@ -162,7 +162,8 @@ int psim_gpu_set_graph(psim_ctx *ctx, int steps_per_graph);
 int psim_gpu_get_params(psim_ctx *ctx, psim_params *out);
 
 /* The pair kernel the context runs: *path = 1 thread per particle, 2 cell
- * per workgroup, 3 brick of cells per workgroup; brick (may be NULL) gets
+ * kernel (a workgroup per cell, or a wave per cell at two to 3.5 particles per
+ * cell: the same results), 3 brick of cells per workgroup; brick (may be NULL) gets
  * the brick's home cells along x, y, z (0 unless path 3) and lanes per
  * particle.  No reference counterpart (the reference has one CPU loop). */
 int psim_gpu_kernel_info(psim_ctx *ctx, int *path, int brick[4]);

@@ -20,6 +20,9 @@
 // workgroup) against five at the compiler's own choice: 137 / 151 us a step at
 // N = 200,000, three per cell.  The workgroup kernel: 210.
 //
+// With ST = NbrStats the accepted pairs are recorded instead (the acceptance
+// code of the forces).
+//
 // Cells it is not made for (more than kCellHome particles, fewer than 4 or
 // more than kCellCap candidates, more than kCellPairs pairs) are left to the
 // workgroup, which does them the other kernel's way afterwards.
@@ -36,7 +39,9 @@ constexpr int kCellPairs = 128;
 constexpr int kCellMasks = (kCellCap + 63) / 64;
 static_assert(kDenseThreads == 256, "the order of the sums");
 
+// flags of an entry of the pair list
 constexpr int kNewGroup = 0x8000;   // not the group of the pair before
+constexpr int kNoPair = 0x4000;     // not inside the cutoff (statistics)
 
 struct CellShared {
     double s[3][kCellCap];    // candidates, shifted to the home cell's image
@@ -51,12 +56,13 @@ struct CellShared {
 };
 
 // Forces on the home particles of cell c by one wave; epi(slot, fx, fy, fz)
-// takes them.  False, with nothing done, where the cell does not fit.
-template <int MASK, int LJN, class Epi>
+// takes them, or with statistics *so.  False, with nothing done, where the cell
+// does not fit.
+template <int MASK, int LJN, class ST, class Epi>
 __device__ bool cell_forces(const Geo &g, const Pot &p, double radius,
                             const double *__restrict__ pos, const int *__restrict__ cstart,
                             const int *__restrict__ id, DevErr *err, int c, CellShared &sh,
-                            const double *etab, Epi epi)
+                            const double *etab, Epi epi, const NbrStatsOut *so)
 {
     const int N = g.n, S = g.S;
     const int lane = threadIdx.x & 63;
@@ -169,8 +175,10 @@ __device__ bool cell_forces(const Geo &g, const Pot &p, double radius,
     for (int e = lane; e < total; e += 64) {
         const int ent = sh.list[e];
         const int i = ent >> 8, v = ent & 255;
-        const int gp = e ? sh.group[sh.list[e - 1] & 255] : -1;
-        if (gp != sh.group[v]) sh.list[e] = (unsigned short)(ent | kNewGroup);
+        if constexpr (!ST::kOn) {
+            const int gp = e ? sh.group[sh.list[e - 1] & 255] : -1;
+            if (gp != sh.group[v]) sh.list[e] = (unsigned short)(ent | kNewGroup);
+        }
         const double xi = sh.h[0][i], yi = sh.h[1][i], zi = sh.h[2][i];
         const double dx = sh.s[0][v] - xi, dy = sh.s[1][v] - yi, dz = sh.s[2][v] - zi;
         const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
@@ -180,8 +188,14 @@ __device__ bool cell_forces(const Geo &g, const Pot &p, double radius,
             const double r2x = pbc_dist_ref(xi, yi, zi, pos[sj], pos[N + sj], pos[2 * N + sj],
                                             g.L, g.half_pbc);
             in = !(r2 >= p.rc2_lo) || r2x < p.rc2;
-            if (in && sqrt(r2x) < p.ov_factor * size)
+            if (!ST::kOn && in && sqrt(r2x) < p.ov_factor * size)
                 report_error(err, 7704, id[home0 + i], id[sj]);
+        }
+        if constexpr (ST::kOn) {
+            sh.fr[e] = __longlong_as_double(
+                (long long)(in ? nbr_hash((unsigned)id[sh.slot[v]]) : 0ull));
+            if (!in) sh.list[e] = (unsigned short)(ent | kNoPair);
+            continue;
         }
         const double rinv = rsqrt_nr(r2);
         bool nan_ao = false;
@@ -190,6 +204,20 @@ __device__ bool cell_forces(const Geo &g, const Pot &p, double radius,
         sh.fr[e] = in ? fr : 0.0;
     }
     wave_lds_sync();
+    if constexpr (ST::kOn) {
+        if (lane < ni) {
+            int pairs = 0;
+            unsigned long long hash = 0;
+            for (int e = sh.first[4 * lane]; e < sh.first[4 * lane + 4]; ++e) {
+                pairs += sh.list[e] & kNoPair ? 0 : 1;
+                hash += (unsigned long long)__double_as_longlong(sh.fr[e]);
+            }
+            const int o = id[home0 + lane];
+            so->count[o] = pairs;
+            so->hash[o] = hash;
+        }
+        return true;
+    }
     // ---- add: three lanes (dimensions) per home particle and q, the four q
     // of a particle side by side
     for (int w0 = 0; w0 < 4 * ni; w0 += 20) {
@@ -235,12 +263,12 @@ union CellsShared {
 
 // The cells of one workgroup, one per wave, then those that did not fit by
 // the whole workgroup.
-template <int MASK, int LJN, class Epi>
+template <int MASK, int LJN, class ST = NoStats, class Epi>
 __device__ __forceinline__ void cells_forces(const Geo &g, const Pot &p, double radius,
                                              const double *__restrict__ pos,
                                              const int *__restrict__ cstart,
                                              const int *__restrict__ id, DevErr *err, int per_xcd,
-                                             Epi epi)
+                                             Epi epi, const NbrStatsOut *so = nullptr)
 {
     __shared__ CellsShared sh;
     __shared__ double etab[64];
@@ -250,17 +278,17 @@ __device__ __forceinline__ void cells_forces(const Geo &g, const Pot &p, double 
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int c = xcd_cell(blockIdx.x, per_xcd) * (kCellBlock / 64) + w;
     const bool done = c >= g.ncell ||
-                      cell_forces<MASK, LJN>(g, p, radius, pos, cstart, id, err, c, sh.w[w],
-                                             etab, epi);
+                      cell_forces<MASK, LJN, ST>(g, p, radius, pos, cstart, id, err, c, sh.w[w],
+                                                 etab, epi, so);
     if ((threadIdx.x & 63) == 0) left[w] = done ? -1 : c;
     __syncthreads();
     for (int k = 0; k < kCellBlock / 64; ++k) {
         const int q = left[k];
         if (q < 0) continue;
         const int home0 = cstart[q];
-        dense_cell_forces<MASK, kDenseThreads, LJN>(
+        dense_cell_forces<MASK, kDenseThreads, LJN, ST>(
             g, p, radius, pos, cstart, id, err, q, sh.d,
-            [=](int i, double fx, double fy, double fz) { epi(home0 + i, fx, fy, fz); });
+            [=](int i, double fx, double fy, double fz) { epi(home0 + i, fx, fy, fz); }, so);
     }
 }
 

@@ -285,7 +285,11 @@ void launch_forces_mask(psim_ctx *c)
 // Neighbour-set statistics with the launch shape launch_step_mask uses.
 void launch_stats(psim_ctx *c, NbrStatsOut so)
 {
-    if (c->dense) {
+    if (c->cells) {
+        const int per = cells_per_xcd(c->ncell);
+        k_stats_cells<<<8 * per, kCellBlock, 0, c->stream>>>(c->geo, c->pot, c->prm.radius,
+                                                             c->pos, c->id, c->cstart, so, per);
+    } else if (c->dense) {
         const int per = (c->ncell + 7) / 8;
         k_stats_dense<<<8 * per, kDenseThreads, 0, c->stream>>>(c->geo, c->pot, c->prm.radius,
                                                                 c->pos, c->id, c->cstart, so,

@@ -478,7 +478,7 @@ inline int cells_per_xcd(int ncell)
 // ---------------------------------------------------------------------------
 // Neighbour-set statistics of the pair kernels: the launch shapes and the
 // acceptance code of the step kernels (k_step with BLOCK / SPLIT,
-// k_step_dense, k_step_brick with G), each accepted pair recorded in an
+// k_step_dense, k_step_cells, k_step_brick with G), each accepted pair recorded in an
 // NbrStats instead of evaluated; counts and partner hashes by original index.
 // ---------------------------------------------------------------------------
 template <int BLOCK, int SPLIT>
@@ -517,6 +517,15 @@ __attribute__((amdgpu_waves_per_eu(dense_waves(F_CAL)))) void k_stats_dense(
     if (c >= g.ncell) return;
     dense_cell_forces<F_CAL, kDenseThreads, 0, NbrStats>(
         g, p, radius, pos, cstart, id, nullptr, c, sh, [](int, double, double, double) {}, &so);
+}
+
+__global__ __launch_bounds__(kCellBlock)
+__attribute__((amdgpu_waves_per_eu(cell_waves(F_CAL)))) void k_stats_cells(
+    Geo g, Pot p, double radius, const double *pos, const int *id, const int *cstart,
+    NbrStatsOut so, int per_xcd)
+{
+    cells_forces<F_CAL, 0, NbrStats>(g, p, radius, pos, cstart, id, nullptr, per_xcd,
+                                     [](int, double, double, double) {}, &so);
 }
 
 template <int G>
