@@ -113,16 +113,26 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_reduce(const int *count, 
     }
 }
 
-// The tile totals replaced by their exclusive prefix sums (one block).
+// The tile totals replaced by their exclusive prefix sums (one block, eight
+// totals per thread and round).
 __global__ __launch_bounds__(kScanThreads) void k_scan_bsum(int *bsum, int nb)
 {
+    constexpr int kItems = 8;
     int carry = 0;
-    for (int b0 = 0; b0 < nb; b0 += kScanThreads) {
-        const int i = b0 + (int)threadIdx.x;
-        const int v = i < nb ? bsum[i] : 0;
+    for (int b0 = 0; b0 < nb; b0 += kItems * kScanThreads) {
+        const int i = b0 + kItems * (int)threadIdx.x;
+        int v[kItems], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) v[k] = i + k < nb ? bsum[i + k] : 0;
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) sum += v[k];
         int total;
-        const int pre = block_exclusive_scan(v, &total);
-        if (i < nb) bsum[i] = carry + pre;
+        int pre = carry + block_exclusive_scan(sum, &total);
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) {
+            if (i + k < nb) bsum[i + k] = pre;
+            pre += v[k];
+        }
         carry += total;
     }
 }
@@ -269,12 +279,33 @@ struct Rebuilt {
     int *id2, *inv2;
 };
 
-constexpr int kTileThreads = 256;
+constexpr int kTileList = 1024;   // members in LDS at a time
+
+// The particle of slot s (position, original id o) to slot dst of cell c.
+template <class Box>
+__device__ __forceinline__ void put_particle(const Rebuilt &to, int n, int dst, int s, double px,
+                                             double py, double pz, int o, int c, const Box &box)
+{
+    to.pos[dst] = px;
+    to.pos[n + dst] = py;
+    to.pos[2 * n + dst] = pz;
+    if (to.pos2) {
+        to.pos2[dst] = px;
+        to.pos2[n + dst] = py;
+        to.pos2[2 * n + dst] = pz;
+    }
+    if (Box::kPack) to.upos[dst] = pack_position(px, py, pz, c, box(dst));
+    to.id[dst] = o;
+    if (to.id2) to.id2[dst] = o;
+    if (to.inv2) to.inv2[o] = dst;
+    to.prev[dst] = s;
+}
 
 // The cell rebuild in one launch: start table, canonical order, positions and
 // ids moved into it.
 //
-// A workgroup owns a tile of 1 << shift consecutive cells.  Its first slot is
+// A workgroup owns a tile of 1 << shift consecutive cells, at most kPer per
+// thread.  Its first slot is
 // the sum of the tile totals before it (prefixed: tile_total already holds
 // that sum), the starts of its cells a scan of their counts; the members come
 // from the cells' bins, and a member's place in its cell is the number of
@@ -292,9 +323,15 @@ constexpr int kTileThreads = 256;
 // 262,144 AO particles, now a step of 33.3; 19.1 for 23.0 us at 4,096 (three
 // kernels before), 27.4 for 36.0 at 30,011, 829 for 900 at 2,097,152.
 //
-// Each lane moves up to U particles with their loads together; a tile with
-// more members than U * kTileThreads keeps its list in perm (which has room
-// for it at the tile's slots) instead of LDS and goes round by round.
+// Each lane moves up to U particles with their loads together.  A tile with
+// more members than U * kTileThreads (a dense spot) is done in batches of
+// cells that fit the list, kWide particles per lane; a cell that does not fit
+// by itself keeps its members in perm, which has room for them at the cell's
+// slots.
+//
+// split: the kernel stops at the start table and the chains (left in perm), and
+// k_place moves the particles, one per lane over the whole grid: see
+// shape_bins.
 //
 // The kernel clears what the next step counts into: the counts of its cells,
 // the heads of its chains, and next_total, the other of two arrays of tile
@@ -303,17 +340,17 @@ constexpr int kTileThreads = 256;
 // the clock and the next step's flags, which no kernel of this step reads
 // after the integrator.  Box::kPack: the new positions' box fractions and
 // cells are written to upos too (the thread-per-particle kernels' cull).
-template <int U, class Box>
+template <int U, int kPer, class Box>
 __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins b, int prefixed,
-                                                          int *next_total, int *perm,
+                                                          int split, int *next_total, int *perm,
                                                           const double *__restrict__ npos,
                                                           const int *__restrict__ id_in,
                                                           StepCtl *ctl, Box box, Rebuilt to)
 {
-    constexpr int kList = U * kTileThreads;
-    __shared__ int start[kTileCells + 1];
-    __shared__ int list[kList];
-    __shared__ unsigned short cell_of[kList];
+    constexpr int kDirect = U * kTileThreads;
+    __shared__ int start[kPer * kTileThreads + 1];
+    __shared__ int list[kTileList];
+    __shared__ unsigned short cell_of[kTileList];
     __shared__ int wsum[2][kTileThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // below the size of U = 4 a tile runs on the XCD whose L2 the integrator
@@ -337,26 +374,31 @@ __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins
                       (i + 3 < tile ? q.w : 0);
         }
     }
-    const int k0 = tid * 4;
-    int cnt[4] = {0, 0, 0, 0};
-    if (k0 + 4 <= cells) {
-        int4 *p = reinterpret_cast<int4 *>(b.count + c0 + k0);
-        const int4 q = *p;
-        cnt[0] = q.x;
-        cnt[1] = q.y;
-        cnt[2] = q.z;
-        cnt[3] = q.w;
-        *p = make_int4(0, 0, 0, 0);
-    } else {
+    const int k0 = tid * kPer;
+    int cnt[kPer] = {};
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (k0 + k < cells) {
-                cnt[k] = b.count[c0 + k0 + k];
-                b.count[c0 + k0 + k] = 0;
-            }
+    for (int k = 0; k < kPer; k += 4) {
+        if (k0 + k + 4 <= cells) {
+            int4 *p = reinterpret_cast<int4 *>(b.count + c0 + k0 + k);
+            const int4 q = *p;
+            cnt[k] = q.x;
+            cnt[k + 1] = q.y;
+            cnt[k + 2] = q.z;
+            cnt[k + 3] = q.w;
+            *p = make_int4(0, 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int u = k; u < k + 4; ++u)
+                if (k0 + u < cells) {
+                    cnt[u] = b.count[c0 + k0 + u];
+                    b.count[c0 + k0 + u] = 0;
+                }
+        }
     }
     if (tid == 0) next_total[tile] = 0;
-    const int mine = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    int mine = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) mine += cnt[k];
     int x = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -376,27 +418,34 @@ __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins
         m += wsum[0][v];
         base += wsum[1][v];
     }
-    const bool fits = m <= kList;
+    const bool direct = m <= kDirect && !split;
     {
-        const int st[4] = {pre, pre + cnt[0], pre + cnt[0] + cnt[1], pre + cnt[0] + cnt[1] + cnt[2]};
+        int st[kPer];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < kPer; ++k) {
+            st[k] = pre;
+            pre += cnt[k];
             if (k0 + k < cells) {
                 start[k0 + k] = st[k];
-                if (fits)
+                if (direct)
                     for (int j = 0; j < cnt[k]; ++j) cell_of[st[k] + j] = (unsigned short)(k0 + k);
             }
-        if (k0 + 4 <= cells) {
-            const int4 q = make_int4(base + st[0], base + st[1], base + st[2], base + st[3]);
-            *reinterpret_cast<int4 *>(to.cstart + c0 + k0) = q;
-        } else {
+        }
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (k0 + k < cells) to.cstart[c0 + k0 + k] = base + st[k];
+        for (int k = 0; k < kPer; k += 4) {
+            if (k0 + k + 4 <= cells) {
+                const int4 q = make_int4(base + st[k], base + st[k + 1], base + st[k + 2],
+                                         base + st[k + 3]);
+                *reinterpret_cast<int4 *>(to.cstart + c0 + k0 + k) = q;
+            } else {
+#pragma unroll
+                for (int u = k; u < k + 4; ++u)
+                    if (k0 + u < cells) to.cstart[c0 + k0 + u] = base + st[u];
+            }
         }
         if (to.cstart2) {   // of any alignment
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < kPer; ++k)
                 if (k0 + k < cells) to.cstart2[c0 + k0 + k] = base + st[k];
         }
     }
@@ -410,56 +459,55 @@ __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins
     __syncthreads();
     if (m == 0) return;
 
-    // member j of the tile (cell i, r-th of its bin) into the list; the first
-    // member past the row walks the cell's chain
+    // chain q of cell i: members cap + q, cap + q + kChains, ... to out[0],
+    // out[kChains], ...
+    auto unchain = [&](int i, int q, int *out) {
+        int *head = b.over + (size_t)n + (size_t)(c0 + i) * kChains + q;
+        int s = *head;
+        *head = -1;
+        const int end = start[i + 1] - start[i] - b.cap - q;
+        for (int k = 0; k < end && s >= 0; k += kChains) {
+            out[k] = s;
+            s = b.over[s];
+        }
+    };
+    if (split) {
+        for (int t = tid; t < cells * kChains; t += kTileThreads) {
+            const int i = t / kChains, q = t % kChains;
+            if (start[i + 1] - start[i] > b.cap + q) unchain(i, q, perm + base + start[i] + b.cap + q);
+        }
+        return;
+    }
+    // member j of the tile (cell i, r-th of its bin) to *out; the first members
+    // past the row walk the cell's chains
     auto fetch = [&](int j, int i, int *out) {
         const int r = j - start[i];
-        const int c = c0 + i;
         if (r < b.cap) {
-            const int s = b.tab[(size_t)c * b.cap + r];
-            out[j] = s;
+            const int s = *b.place(c0 + i, r);
+            *out = s;
             return s;
         }
-        if (r == b.cap) {
-            int *head = b.over + (size_t)n + c;
-            int s = *head;
-            *head = -1;
-            for (int q = j; q < start[i + 1] && s >= 0; ++q) {
-                out[q] = s;
-                s = b.over[s];
-            }
-        }
+        if (r < b.cap + kChains) unchain(i, r - b.cap, out);
         return -1;
     };
     auto place = [&](int i, int rank, int s, double px, double py, double pz, int o) {
-        const int dst = base + start[i] + rank;
-        to.pos[dst] = px;
-        to.pos[n + dst] = py;
-        to.pos[2 * n + dst] = pz;
-        if (to.pos2) {
-            to.pos2[dst] = px;
-            to.pos2[n + dst] = py;
-            to.pos2[2 * n + dst] = pz;
-        }
-        if (Box::kPack) to.upos[dst] = pack_position(px, py, pz, c0 + i, box(dst));
-        to.id[dst] = o;
-        if (to.id2) to.id2[dst] = o;
-        if (to.inv2) to.inv2[o] = dst;
-        to.prev[dst] = s;
+        put_particle(to, n, base + start[i] + rank, s, px, py, pz, o, c0 + i, box);
     };
+    // l: the members of cell i
     auto rank_in = [&](const int *l, int i, int s) {
+        const int len = start[i + 1] - start[i];
         int rank = 0;
-        for (int k = start[i]; k < start[i + 1]; ++k) rank += l[k] < s;
+        for (int k = 0; k < len; ++k) rank += l[k] < s;
         return rank;
     };
-    if (fits) {
+    if (direct) {
         int i[U], s[U], o[U];
         double p[U][3];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int j = tid + u * kTileThreads;
             i[u] = j < m ? cell_of[j] : 0;
-            s[u] = j < m ? fetch(j, i[u], list) : -1;
+            s[u] = j < m ? fetch(j, i[u], list + j) : -1;
         }
         __syncthreads();
 #pragma unroll
@@ -473,30 +521,137 @@ __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (tid + u * kTileThreads < m)
-                place(i[u], rank_in(list, i[u], s[u]), s[u], p[u][0], p[u][1], p[u][2], o[u]);
-    } else {
-        auto cell = [&](int j) {   // the last cell that starts at or before j
-            int lo = 0, hi = cells - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (start[mid] <= j) lo = mid; else hi = mid - 1;
+                place(i[u], rank_in(list + start[i[u]], i[u], s[u]), s[u], p[u][0], p[u][1],
+                      p[u][2], o[u]);
+        return;
+    }
+    // Batches of cells whose members fit the list: kWide members per lane, their
+    // searches and loads together, and kDeep members of each one's cell at a
+    // time for its rank (four and two, or four and four: no faster, 79 and 86
+    // VGPRs instead of 50).  A drop of 160,000 LJ particles, 12 to 27 per cell,
+    // in 40,000 of vapour: the rebuild takes 38 us, 101 with the members and
+    // their order in global memory, 10 to 22 without the drop.
+    constexpr int kWide = 2, kDeep = 4;
+    auto last_at = [&](int j, int lo, int hi) {   // last of lo..hi that starts at or before j
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (start[mid] <= j) lo = mid; else hi = mid - 1;
+        }
+        return lo;
+    };
+    // l: the members of cells i0 .. i1 - 1
+    auto batch = [&](int i0, int i1, int *l, bool in_list) __attribute__((always_inline)) {
+        const int j0 = start[i0], j1 = start[i1];
+        int top = 1;
+        while (top < i1 - i0) top *= 2;
+        for (int j = j0 + tid; j < j1; j += kWide * kTileThreads) {
+            int i[kWide];
+#pragma unroll
+            for (int u = 0; u < kWide; ++u) i[u] = i0;
+            for (int step = top >> 1; step; step >>= 1)
+#pragma unroll
+                for (int u = 0; u < kWide; ++u) {
+                    const int mid = min(i[u] + step, i1 - 1);
+                    if (start[mid] <= j + u * kTileThreads) i[u] = mid;
+                }
+#pragma unroll
+            for (int u = 0; u < kWide; ++u) {
+                const int q = j + u * kTileThreads;
+                if (q < j1) {
+                    fetch(q, i[u], l + (q - j0));
+                    if (in_list) cell_of[q - j0] = (unsigned short)i[u];
+                }
             }
-            return lo;
-        };
-        int *l = perm + base;
-        for (int j = tid; j < m; j += kTileThreads) fetch(j, cell(j), l);
+        }
         __syncthreads();
-        for (int j = tid; j < m; j += kTileThreads) {
-            const int s = l[j], i = cell(j);
-            place(i, rank_in(l, i, s), s, npos[s], npos[n + s], npos[2 * n + s], id_in[s]);
+        for (int j = j0 + tid; j < j1; j += kWide * kTileThreads) {
+            int s[kWide], o[kWide], at[kWide], len[kWide], rank[kWide], i[kWide], most = 0;
+            double p[kWide][3];
+#pragma unroll
+            for (int u = 0; u < kWide; ++u) {   // (a missing member repeats the last)
+                const int q = min(j + u * kTileThreads, j1 - 1) - j0;
+                s[u] = l[q];
+                i[u] = in_list ? cell_of[q] : i0;
+            }
+#pragma unroll
+            for (int u = 0; u < kWide; ++u) {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) p[u][d] = npos[d * n + s[u]];
+                o[u] = id_in[s[u]];
+                at[u] = start[i[u]] - j0;
+                len[u] = start[i[u] + 1] - start[i[u]];
+                rank[u] = 0;
+                most = max(most, len[u]);
+            }
+            for (int k = 0; k < most; k += kDeep)
+#pragma unroll
+                for (int u = 0; u < kWide; ++u)
+#pragma unroll
+                    for (int q = 0; q < kDeep; ++q)
+                        rank[u] += (k + q < len[u]) & (l[min(at[u] + k + q, j1 - j0 - 1)] < s[u]);
+#pragma unroll
+            for (int u = 0; u < kWide; ++u)
+                if (j + u * kTileThreads < j1)
+                    place(i[u], rank[u], s[u], p[u][0], p[u][1], p[u][2], o[u]);
+        }
+        __syncthreads();   // the list is free again
+    };
+    for (int i0 = 0; i0 < cells;) {
+        const int i1 = last_at(start[i0] + kTileList, i0, cells);
+        if (i1 > i0) {
+            batch(i0, i1, list, true);
+            i0 = i1;
+        } else {
+            batch(i0, i0 + 1, perm + base + start[i0], false);
+            ++i0;
         }
     }
 }
 
-// A workgroup sums the totals before its tile itself up to this many tiles
-// (eight loads of 16 bytes per lane); beyond that one block turns them into
-// prefixes first.
-constexpr int kSelfPrefixTiles = 8192;
+// The other half of a split rebuild: the particle of every slot of the bins'
+// order (cell by cell, rows and then chains) to its place in its cell.  Each
+// lane finds its cell in the start table.
+template <class Box>
+__global__ __launch_bounds__(256) void k_place(int n, int ncell, Bins b,
+                                               const int *__restrict__ perm,
+                                               const double *__restrict__ npos,
+                                               const int *__restrict__ id_in, Box box, Rebuilt to)
+{
+    const int t = xcd_block() * 256 + threadIdx.x;
+    if (t >= n) return;
+    int c = 0;
+    for (int hi = ncell - 1; c < hi;) {
+        const int mid = c + (hi - c + 1) / 2;
+        if (to.cstart[mid] <= t) c = mid; else hi = mid - 1;
+    }
+    const int base = to.cstart[c], len = to.cstart[c + 1] - base;
+    const int *row = b.place(c, 0);
+    const int s = t - base < b.cap ? row[t - base] : perm[t];
+    const double x = npos[s], y = npos[n + s], z = npos[2 * n + s];
+    const int o = id_in[s];
+    // (16 members' loads in flight; a row is a multiple of 16 long here)
+    const int in_row = min(len, b.cap);
+    int rank = 0;
+    for (int r = 0; r < in_row; r += 16) {
+        int4 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = reinterpret_cast<const int4 *>(row + r)[q];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = r + 4 * q;
+            rank += (k < in_row && v[q].x < s) + (k + 1 < in_row && v[q].y < s) +
+                    (k + 2 < in_row && v[q].z < s) + (k + 3 < in_row && v[q].w < s);
+        }
+    }
+    for (int k = in_row; k < len; ++k) rank += perm[base + k] < s;
+    put_particle(to, n, base + rank, s, x, y, z, o, c, box);
+}
+
+// A workgroup sums the totals before its tile itself up to this many tiles (16
+// loads of 16 bytes per lane); beyond that one block turns them into prefixes
+// first.  (10,044 tiles, a step at N = 262,144 in 20.6 million cells: 126.5 us
+// with the prefix launch, 115.1 without.)
+constexpr int kSelfPrefixTiles = 16384;
 
 template <class Box>
 void launch_rebuild(hipStream_t st, int n, int ncell, BinStore &t, const double *npos,
@@ -504,15 +659,21 @@ void launch_rebuild(hipStream_t st, int n, int ncell, BinStore &t, const double 
 {
     const int prefixed = t.tiles > kSelfPrefixTiles;
     if (prefixed) k_scan_bsum<<<1, kScanThreads, 0, st>>>(t.b.tile_total, t.tiles);
-    auto go = [&](auto u) {
-        k_rebuild<decltype(u)::value><<<decltype(u)::value < 4 ? xcd_grid(t.tiles) : t.tiles, kTileThreads, 0, st>>>(
-            n, ncell, t.b, prefixed, t.next_total, t.perm, npos, id_in, ctl, box, to);
+    auto go = [&](auto lanes, auto per) {
+        constexpr int kU = decltype(lanes)::value;
+        k_rebuild<kU, decltype(per)::value>
+            <<<kU < 4 ? xcd_grid(t.tiles) : t.tiles, kTileThreads, 0, st>>>(
+                n, ncell, t.b, prefixed, t.split, t.next_total, t.perm, npos, id_in, ctl, box, to);
     };
-    switch (t.lanes) {
-    case 4: go(std::integral_constant<int, 4>{}); break;
-    case 2: go(std::integral_constant<int, 2>{}); break;
-    default: go(std::integral_constant<int, 1>{}); break;
-    }
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    const std::integral_constant<int, 8> eight;
+    if (t.per == 8) t.lanes == 4 ? go(four, eight) : t.lanes == 2 ? go(two, eight) : go(one, eight);
+    else t.lanes == 4 ? go(four, four) : t.lanes == 2 ? go(two, four) : go(one, four);
+    if (t.split)
+        k_place<<<xcd_grid((n + 255) / 256), 256, 0, st>>>(n, ncell, t.b, t.perm, npos, id_in, box,
+                                                           to);
 }
 
 // The lagged arrays (previous positions, last forces, memory, kept in the

@@ -422,14 +422,22 @@ __device__ __forceinline__ void wave_count(int *tile_total, int t)
     }
 }
 
+constexpr int kChains = 4;   // of a cell (walked side by side)
+
 // What a step's integrator leaves for the cell rebuild: the members of every
 // cell in any order and the totals of the tiles of 1 << shift cells.
 struct Bins {
     int *count;        // [cells] members; the rebuild clears it
-    int *tab;          // [cells][cap] slots of the first cap members
-    int *over;         // [n] next, [cells] head: the members past cap as chains
+    int *tab;          // slots of the first cap members: member r of cell c at
+                       // c * cell_step + r * member_step
+    int *over;         // [n] next, [cells][kChains] head: the members past cap as
+                       // chains, dealt round
     int *tile_total;   // [tiles]
-    int cap, shift;
+    int cap, shift, cell_step, member_step;
+    __device__ __forceinline__ int *place(int c, int r) const
+    {
+        return tab + ((size_t)c * (unsigned)cell_step + (size_t)r * (unsigned)member_step);
+    }
 };
 
 // The particle of slot s goes to cell c (n particles in all).
@@ -438,9 +446,9 @@ __device__ __forceinline__ void bin_particle(const Bins &b, int n, int s, int c)
     wave_count(b.tile_total, c >> b.shift);
     const int r = wave_aggregated_rank(b.count, c);
     if (r < b.cap)
-        b.tab[(size_t)c * b.cap + r] = s;
+        *b.place(c, r) = s;
     else
-        b.over[s] = atomicExch(&b.over[(size_t)n + c], s);
+        b.over[s] = atomicExch(&b.over[(size_t)n + (size_t)c * kChains + (r - b.cap) % kChains], s);
 }
 
 // ---------------------------------------------------------------------------
