@@ -25,7 +25,10 @@ struct BinStore {
 //
 // A bin holds what hard particles can pack into a cell, or four times the mean
 // and a few (at least 32), whichever is less; a longer chain costs time, not
-// correctness.  The bins lie member by member (all first members, all second
+// correctness.  Bins that would take more than 256 bytes per particle and more
+// than 1 GiB (boxes with hardly any particle per cell) are made shorter, down to
+// one member, and have one chain per cell instead of four: at 1290^3 cells, the
+// most there are, 12 bytes per cell beside the start table.  The bins lie member by member (all first members, all second
 // ones, ...): the lines that a dilute system touches are full of what its
 // neighbours wrote.  With a row per cell a step at N = 1,200,000 in 4.1 million
 // cells took 168 us (now 139), at 2,097,152 AO in 40 million 531 (488), at
@@ -59,6 +62,12 @@ inline void shape_bins(int n, int ncell, double cell_volume, BinStore &t)
     const double most = fmin(fmax(packed, 2.0 * occ + 2.0), (double)n);
     t.b.cap = t.split ? 16 : 4;   // (rows are read 16 at a time)
     while (t.b.cap < most) t.b.cap *= 2;
+    t.b.chains = 4;
+    const double room = fmax(256.0 * n, 1073741824.0);
+    while (t.b.cap > 1 && 4.0 * ncell * t.b.cap > room) {
+        t.b.cap /= 2;
+        t.b.chains = 1;
+    }
     t.b.cell_step = t.split ? t.b.cap : 1;
     t.b.member_step = t.split ? 1 : ncell;
     const double members = t.lanes > 1 ? 192.0 * t.lanes : fmin(fmax(n / 256.0, 64.0), 192.0);
@@ -73,7 +82,7 @@ int alloc_bins(int n, int ncell, BinStore &t, Alloc alloc)
 {
     int rc = alloc(&t.b.count, (size_t)ncell);
     if (!rc) rc = alloc(&t.b.tab, (size_t)ncell * t.b.cap);
-    if (!rc) rc = alloc(&t.b.over, (size_t)n + (size_t)ncell * kChains);
+    if (!rc) rc = alloc(&t.b.over, (size_t)n + (size_t)ncell * t.b.chains);
     if (!rc) rc = alloc(&t.b.tile_total, (size_t)t.tiles + 3);   // read by fours
     if (!rc) rc = alloc(&t.next_total, (size_t)t.tiles + 3);
     if (!rc) rc = alloc(&t.perm, (size_t)n);
@@ -91,7 +100,7 @@ inline hipError_t clear_bins(hipStream_t st, int n, int ncell, const BinStore &t
 {
     const size_t tb = sizeof(int) * ((size_t)t.tiles + 3);
     hipError_t e = hipMemsetAsync(t.b.count, 0, sizeof(int) * ncell, st);
-    if (e == hipSuccess) e = hipMemsetAsync(t.b.over + n, 0xff, sizeof(int) * kChains * ncell, st);
+    if (e == hipSuccess) e = hipMemsetAsync(t.b.over + n, 0xff, sizeof(int) * t.b.chains * ncell, st);
     if (e == hipSuccess) e = hipMemsetAsync(t.b.tile_total, 0, tb, st);
     if (e == hipSuccess) e = hipMemsetAsync(t.next_total, 0, tb, st);
     return e;

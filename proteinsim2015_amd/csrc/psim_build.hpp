@@ -459,23 +459,22 @@ __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins
     __syncthreads();
     if (m == 0) return;
 
-    // chain q of cell i: members cap + q, cap + q + kChains, ... to out[0],
-    // out[kChains], ...
+    // chain q of cell i: members cap + q, cap + q + chains, ... to out[0],
+    // out[chains], ...
     auto unchain = [&](int i, int q, int *out) {
-        int *head = b.over + (size_t)n + (size_t)(c0 + i) * kChains + q;
+        int *head = b.over + (size_t)n + (size_t)(c0 + i) * b.chains + q;
         int s = *head;
         *head = -1;
         const int end = start[i + 1] - start[i] - b.cap - q;
-        for (int k = 0; k < end && s >= 0; k += kChains) {
+        for (int k = 0; k < end && s >= 0; k += b.chains) {
             out[k] = s;
             s = b.over[s];
         }
     };
     if (split) {
-        for (int t = tid; t < cells * kChains; t += kTileThreads) {
-            const int i = t / kChains, q = t % kChains;
-            if (start[i + 1] - start[i] > b.cap + q) unchain(i, q, perm + base + start[i] + b.cap + q);
-        }
+        for (int i = tid; i < cells; i += kTileThreads)
+            for (int q = 0; q < b.chains && start[i + 1] - start[i] > b.cap + q; ++q)
+                unchain(i, q, perm + base + start[i] + b.cap + q);
         return;
     }
     // member j of the tile (cell i, r-th of its bin) to *out; the first members
@@ -487,7 +486,7 @@ __global__ __launch_bounds__(kTileThreads) void k_rebuild(int n, int ncell, Bins
             *out = s;
             return s;
         }
-        if (r < b.cap + kChains) unchain(i, r - b.cap, out);
+        if (r < b.cap + b.chains) unchain(i, r - b.cap, out);
         return -1;
     };
     auto place = [&](int i, int rank, int s, double px, double py, double pz, int o) {

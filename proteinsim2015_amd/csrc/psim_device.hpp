@@ -422,18 +422,16 @@ __device__ __forceinline__ void wave_count(int *tile_total, int t)
     }
 }
 
-constexpr int kChains = 4;   // of a cell (walked side by side)
-
 // What a step's integrator leaves for the cell rebuild: the members of every
 // cell in any order and the totals of the tiles of 1 << shift cells.
 struct Bins {
     int *count;        // [cells] members; the rebuild clears it
     int *tab;          // slots of the first cap members: member r of cell c at
                        // c * cell_step + r * member_step
-    int *over;         // [n] next, [cells][kChains] head: the members past cap as
-                       // chains, dealt round
+    int *over;         // [n] next, [cells][chains] head: the members past cap as
+                       // chains (a power of two, walked side by side), dealt round
     int *tile_total;   // [tiles]
-    int cap, shift, cell_step, member_step;
+    int cap, chains, shift, cell_step, member_step;
     __device__ __forceinline__ int *place(int c, int r) const
     {
         return tab + ((size_t)c * (unsigned)cell_step + (size_t)r * (unsigned)member_step);
@@ -448,7 +446,8 @@ __device__ __forceinline__ void bin_particle(const Bins &b, int n, int s, int c)
     if (r < b.cap)
         *b.place(c, r) = s;
     else
-        b.over[s] = atomicExch(&b.over[(size_t)n + (size_t)c * kChains + (r - b.cap) % kChains], s);
+        b.over[s] = atomicExch(
+            &b.over[(size_t)n + (size_t)c * b.chains + ((r - b.cap) & (b.chains - 1))], s);
 }
 
 // ---------------------------------------------------------------------------

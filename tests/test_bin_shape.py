@@ -20,8 +20,8 @@ int main() {
     while (std::scanf("%d %lld %lf", &n, &ncell, &volume) == 3) {
         psim::BinStore t;
         psim::shape_bins(n, (int)ncell, volume, t);
-        std::printf("%d %d %d %d %d %d %d %d\n", t.lanes, t.per, (int)t.split, t.b.cap, t.b.cell_step,
-                    t.b.member_step, t.b.shift, t.tiles);
+        std::printf("%d %d %d %d %d %d %d %d %d\n", t.lanes, t.per, (int)t.split, t.b.cap, t.b.cell_step,
+                    t.b.member_step, t.b.shift, t.tiles, t.b.chains);
     }
 }
 """
@@ -54,7 +54,7 @@ def shapes(tmp_path_factory):
 
 
 def test_tiles_cover_the_cells(shapes):
-    for (n, ncell, _), (lanes, per, split, cap, cell_step, member_step, shift, tiles) in shapes:
+    for (n, ncell, _), (lanes, per, split, cap, cell_step, member_step, shift, tiles, chains) in shapes:
         assert per in (4, 8) and 4 <= 1 << shift <= per * 256
         assert (tiles - 1) << shift < ncell <= tiles << shift
 
@@ -62,19 +62,35 @@ def test_tiles_cover_the_cells(shapes):
 def test_a_mean_tile_is_moved_at_once(shapes):
     """A workgroup moves 256 particles per lane's share at once; where a tile of
     four cells holds more, the rebuild is split."""
-    for (n, ncell, v), (lanes, per, split, cap, cell_step, member_step, shift, tiles) in shapes:
+    for (n, ncell, v), (lanes, per, split, cap, cell_step, member_step, shift, tiles, chains) in shapes:
         mean = n / ncell * (1 << shift)
         assert split or mean <= 256 * lanes, (n, ncell, v)
         assert not split or n / ncell > 50
 
 
 def test_bins_are_addressed_apart(shapes):
-    for (n, ncell, v), (lanes, per, split, cap, cell_step, member_step, shift, tiles) in shapes:
+    for (n, ncell, v), (lanes, per, split, cap, cell_step, member_step, shift, tiles, chains) in shapes:
         assert cap & (cap - 1) == 0
         if split:   # k_place reads whole rows, 16 members at a time
             assert (cell_step, member_step) == (cap, 1) and cap % 16 == 0
         else:
             assert (cell_step, member_step) == (1, ncell)
+
+
+def test_memory_of_dilute_boxes(shapes):
+    """Bins and chain heads stay within 256 bytes per particle or 1 GiB, or come
+    down to 12 bytes per cell (8 bytes per cell is what the tables of counts and
+    starts take by themselves)."""
+    least = 0
+    for (n, ncell, v), (lanes, per, split, cap, cell_step, member_step, shift, tiles, chains) in shapes:
+        assert cap >= 1 and chains in (1, 4)
+        assert cap == 1 or 4 * cap * ncell <= max(256 * n, 1 << 30), (n, ncell, v)
+        if cap == 1 and ncell > 1 << 28:
+            assert chains == 1
+            least += 1
+        if n / ncell > 1:   # the mean fits with room to spare
+            assert cap > n / ncell or cap >= n
+    assert least
 
 
 def test_line_of_the_split_rebuild(shapes):
