@@ -205,10 +205,11 @@ int psim_gpu_pair_stats(psim_ctx *ctx, int which, int *count_by_orig,
  * forbid hipMalloc).  params as for psim_gpu_create; d_pos and d_force are
  * DEVICE arrays of n x 3 doubles by original index; stream is a hipStream_t
  * (NULL: the null stream).  The cell build's working arrays live in a
- * static device array of PSIM_NOALLOC_SCRATCH_BYTES per GPU (held until
- * the process ends), so n and S^3 are bounded: about 40 n + 8 S^3 bytes
- * must fit (else PSIM_E_NOMEM and a message on stderr).  Calls that overlap
- * on one GPU race on that array.  Returns after the forces are written: 0,
+ * static device array of PSIM_NOALLOC_SCRATCH_BYTES per GPU, with another
+ * 27 MB behind it for box fractions, held from the library's load until the
+ * process ends; so n and S^3 are bounded: about 40 n + 8 S^3 bytes must fit the
+ * former (else PSIM_E_NOMEM and a message on stderr).  Calls that overlap on
+ * one GPU race on that array.  Returns after the forces are written: 0,
  * 7704 or 7705 as psim_gpu_forces, or PSIM_E_*.  The forces equal
  * psim_gpu_forces' on a context with the same params and positions. */
 #define PSIM_NOALLOC_SCRATCH_BYTES (64u << 20)
