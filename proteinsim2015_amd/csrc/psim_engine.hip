@@ -698,7 +698,7 @@ int psim_gpu_create(const psim_params *params, psim_ctx **out)
     if (!rc && hipMemsetAsync(c->err, 0, sizeof(DevErr), c->stream) != hipSuccess)
         rc = PSIM_E_HIP;
     // the five arrays of a state, each at an aligned place
-    if (!rc && !stage_reserve(c->stage, 5 * (sizeof(double) * n3 + 64))) rc = PSIM_E_HIP;
+    if (!rc) (void)stage_reserve(c->stage, 5 * (sizeof(double) * n3 + 64));
     if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = PSIM_E_HIP;
     if (rc) {
         psim_gpu_destroy(c);

@@ -717,7 +717,7 @@ int psim_ens_create(const psim_params *common, const psim_replica *reps, int nre
     if (!rc && clear_bins(e->stream, e->ntot, e->ncell, e->bins) != hipSuccess) rc = PSIM_E_HIP;
     if (!rc && hipMemset(e->err, 0, sizeof(DevErr)) != hipSuccess) rc = PSIM_E_HIP;
     // the four arrays of a state, each at an aligned place
-    if (!rc && !stage_reserve(e->stage, 4 * (sizeof(double) * n3 + 64))) rc = PSIM_E_HIP;
+    if (!rc) (void)stage_reserve(e->stage, 4 * (sizeof(double) * n3 + 64));
     if (rc) {
         psim_ens_destroy(e);
         return rc;

@@ -33,6 +33,18 @@ bool ok(hipError_t e, const char *what)
     return false;
 }
 
+// The same copies straight from and to pageable memory (no pinned memory to be
+// had).
+int unstaged(hipStream_t st, const Xfer *x, int nx, hipMemcpyKind kind)
+{
+    const bool up = kind == hipMemcpyHostToDevice;
+    for (int k = 0; k < nx; ++k)
+        if (!ok(hipMemcpyAsync(up ? const_cast<void *>(x[k].dev) : x[k].host,
+                               up ? x[k].host : x[k].dev, x[k].bytes, kind, st), "copy"))
+            return -1;
+    return ok(hipStreamSynchronize(st), "copy") ? 0 : -1;
+}
+
 // What stays in flight after a failure still uses the buffer.
 int fail(hipStream_t st)
 {
@@ -45,21 +57,24 @@ int fail(hipStream_t st)
 bool stage_reserve(HostStage &h, size_t bytes)
 {
     const size_t want = std::min(std::max(bytes, (size_t)4096), 2 * kChunk);
-    if (h.cap >= want) return true;
-    stage_free(h);
+    if (h.cap >= want || h.refused) return h.cap != 0;
     // (powers of two: a caller whose calls grow does not reallocate each time)
     size_t cap = 4096;
     while (cap < want) cap *= 2;
-    if (!ok(hipHostMalloc((void **)&h.buf, cap, hipHostMallocDefault), "hipHostMalloc")) {
-        h.buf = nullptr;
-        return false;
+    HostStage grown;
+    bool made = ok(hipHostMalloc((void **)&grown.buf, cap, hipHostMallocDefault), "hipHostMalloc");
+    if (!made) grown.buf = nullptr;
+    for (hipEvent_t &e : grown.done)
+        made = made && ok(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    if (!made) {   // the smaller buffer, if there is one, takes more rounds
+        (void)hipGetLastError();
+        stage_free(grown);
+        h.refused = true;   // asked for once
+        return h.cap != 0;
     }
-    h.cap = cap;
-    for (hipEvent_t &e : h.done)
-        if (!e && !ok(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate")) {
-            stage_free(h);
-            return false;
-        }
+    grown.cap = cap;
+    stage_free(h);
+    h = grown;
     return true;
 }
 
@@ -78,7 +93,7 @@ int stage_read(HostStage &h, hipStream_t st, const Xfer *x, int nx)
 {
     size_t total = 0;
     for (int k = 0; k < nx; ++k) total += padded(x[k].bytes);
-    if (!stage_reserve(h, total)) return -1;
+    if (!stage_reserve(h, total)) return unstaged(st, x, nx, hipMemcpyDeviceToHost);
     if (total <= h.cap) {   // one round
         size_t at = 0;
         for (int k = 0; k < nx; ++k) {
@@ -125,7 +140,7 @@ int stage_write(HostStage &h, hipStream_t st, const Xfer *x, int nx)
 {
     size_t total = 0;
     for (int k = 0; k < nx; ++k) total += padded(x[k].bytes);
-    if (!stage_reserve(h, total)) return -1;
+    if (!stage_reserve(h, total)) return unstaged(st, x, nx, hipMemcpyHostToDevice);
     const bool once = total <= h.cap;
     const size_t half = once ? 0 : h.cap / 2;
     size_t at = 0;

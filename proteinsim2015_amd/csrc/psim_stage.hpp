@@ -10,10 +10,14 @@ namespace psim {
 
 // A context's pinned buffer, at most 8 MiB: made with the context in the size
 // of its state (pinning 8 MiB takes 0.5 ms, which a first call would pay
-// otherwise), grown where a call needs more, freed with the context.  Used by one call on the context at a time, as the context is.
+// otherwise), grown where a call needs more, freed with the context.  Without
+// pinned memory the copies go through a smaller buffer made before, or straight
+// to pageable memory.  Used by one call on the context at a time, as the context
+// is.
 struct HostStage {
     char *buf = nullptr;
     size_t cap = 0;
+    bool refused = false;   // no more pinned memory to be had
     hipEvent_t done[2] = {nullptr, nullptr};
 };
 
@@ -25,7 +29,7 @@ struct Xfer {
 };
 
 // Room for `bytes`, up to the 8 MiB that longer copies pass through in two
-// halves.
+// halves; false where there is no buffer at all.
 bool stage_reserve(HostStage &h, size_t bytes);
 void stage_free(HostStage &h);
 // device -> host, in stream order after what is enqueued; the arrays are
