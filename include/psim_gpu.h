@@ -120,7 +120,7 @@ typedef struct psim_kernel_times {
                                                     the thread-per-particle path) */
     double integrate_ms; int integrate_launches; /* separate G&B kernel (cell-
                                                     per-workgroup path) */
-    double build_ms;     int build_launches;     /* scan + scatter + reorder */
+    double build_ms;     int build_launches;     /* cell rebuild */
     double total_ms;     int steps;
 } psim_kernel_times;
 

@@ -538,8 +538,13 @@ bool same_forces(const psim_params &a, const psim_params &b)
 int adj_block(const psim_ctx *) { return kAdjBlock; }
 // Lanes per particle: small systems spread each particle's 27 cells over 8
 // lanes, so that every CU gets work and each lane waits on fewer lookups
-// (200 steps of 32,768: 8 lanes 6.69 ms, 4 6.92, 16 7.59); larger ones over 2
-// (20 steps of 300,007: one lane 3.92 ms, two 3.73, four 3.95, eight 4.23).
+// (200 steps of 32,768: 8 lanes 6.69 ms, 4 6.92, 16 7.59); larger ones over 2.
+// A backward step of AO particles in us, one / two / four / eight lanes:
+// 32,768 28 / 20 / 17 / 16, 65,536 31 / 25 / 23 / 26, 131,072 39 / 35 / 42 / 47,
+// 262,143 66 / 70 / 83 / 96, 300,007 90 / 83 / 93 / 112, 1,000,003 267 / 263 /
+// 300 / 363; LJ, 32,768 95 / 60 / 45 / 41, 131,072 125 / 111 / 116 / 118,
+// 400,000 319 / 301 / 305 / 333.  (From 65,536 on the line lies too high; two
+// lanes from there on would change the order of those systems' sums.)
 #ifndef PSIM_ADJ_SPLIT
 #define PSIM_ADJ_SPLIT 8
 #endif

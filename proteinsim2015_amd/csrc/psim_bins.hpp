@@ -28,21 +28,23 @@ struct BinStore {
 // correctness.  Bins that would take more than 256 bytes per particle and more
 // than 1 GiB (boxes with hardly any particle per cell) are made shorter, down to
 // one member, and have one chain per cell instead of four: at 1290^3 cells, the
-// most there are, 12 bytes per cell beside the start table.  The bins lie member by member (all first members, all second
-// ones, ...): the lines that a dilute system touches are full of what its
-// neighbours wrote.  With a row per cell a step at N = 1,200,000 in 4.1 million
-// cells took 168 us (now 139), at 2,097,152 AO in 40 million 531 (488), at
-// 1,200,000 LJ at 1.5 per cell 217 (194); at 15 per cell there is no difference
-// (2,097,152: 724, 720).
+// most there are, 12 bytes per cell beside the start table.  The bins lie member
+// by member (all first members, all second ones, ...): the lines that a dilute
+// system touches are full of what its neighbours wrote.  With a row per cell a
+// step at N = 1,200,000 in 4.1 million cells took 168 us (now 138), at 2,097,152
+// AO in 40 million 531 (488), at 1,200,000 LJ at 1.5 per cell 217 (194); at 15
+// per cell there is no difference (2,097,152: 724, 720).
 //
 // A tile holds the cells of about 1/256 of the particles (a workgroup per
 // compute unit), at least 64 and at most 192 per particle of a lane.  Lanes
-// move two particles from 131,072 on (a step at 262,144: one 35.4 us, two 33.9,
-// four 33.9; at 32,768 two are 10 % slower than one) and four from 1,048,576
-// (2,097,152: one 861 us, two 841, four 829).  Tiles of half or twice as many
-// particles: no difference.  It holds at most 1024 cells, or 2048 where there
-// are more of those tiles than the chip holds twice over and they are nearly
-// empty (2,097,152 AO particles in 40 million cells: 489 / 452 us a step,
+// move two particles from 131,072 on and four from 1,048,576 (a step in us, one /
+// two / four, AO at phi = 0.15: 65,536 19.1 / 20.0 / 24.6, 131,072 29.8 / 30.2 /
+// 34.6, 180,000 39.7 / 38.0 / 40.9, 524,288 59.6 / 53.7 / 53.1, 1,048,576 112 /
+// 96 / 99, 1,400,000 185 / 159 / 154; 15 per cell, 65,536 40.0 / 40.7 / 42.6,
+// 262,144 110 / 106 / 108, 1,048,576 391 / 373 / 368).  Tiles of half or twice as
+// many particles: no difference.  It holds at most 1024 cells, or 2048 where
+// there are more of those tiles than the chip holds twice over and they are
+// nearly empty (2,097,152 AO particles in 40 million cells: 489 / 452 us a step,
 // 100,000 in 7.8 million 47.0 / 39.8; at 2 million cells 1.4 us slower).
 //
 // A tile is four cells at least.  Where that many hold more than its workgroup

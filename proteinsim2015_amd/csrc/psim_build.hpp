@@ -5,8 +5,9 @@
 // Replaces system::hashParticles / sortParticles / clearCells /
 // reorderParticles (systemHandling.cpp:33-85): instead of an O(N log N)
 // comparison sort of (hash, index) tuples every step, each particle is
-// entered in the bin of its new cell during the step, and one kernel turns
-// the bins into a start table and moves the state into cell order.  Within a
+// entered in the bin of its new cell during the step, and one kernel (two in
+// crowded boxes) turns the bins into a start table and moves the state into cell
+// order.  Within a
 // cell the order is the previous slot order (a stable counting sort), which
 // makes every run reproducible bit for bit.  The scan and scatter kernels
 // below serve the rebuilds that start from counts (analysis grid, forces

@@ -130,8 +130,8 @@ inline unsigned blocks_for(long long n, int threads)
 {
     return (unsigned)((n + threads - 1) / threads);
 }
-// counts (already accumulated) -> cstart, scatter, canonical move of the
-// positions and ids (the state arrays become lagged)
+// the bins (already filled) -> start table, positions and ids in canonical
+// order (the state arrays become lagged)
 int launch_build(psim_ctx *c);
 // gather lagged pos0 / frc / mem into the current slot order (no-op when
 // they are in it already)

@@ -20,7 +20,8 @@
 //               sort); positions and ids move into it; the positions the
 //               step started from (pos0 of the next step, re-imaged when
 //               read), the forces and the memory stay where the step had or
-//               wrote them (read through the slot map prev).
+//               wrote them (read through the slot map prev).  In crowded
+//               boxes a second kernel, k_place, does the moving.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

@@ -8,7 +8,7 @@
 //     sort over the global cell keys rebuilds every replica's table at once
 //     and the replicas stay contiguous in slot order.
 // Each step is one launch per kernel stage for all replicas (pair forces,
-// one per occupancy class, then G&B, scan, scatter, reorder), so a step of
+// one per occupancy class, then G&B, cell rebuild), so a step of
 // 512 replicas costs a handful of launches, and the sequence can be captured
 // once in a hipGraph and replayed.  The step counter, time and velocity-step
 // flags live in device memory (StepCtl) so replays advance them.

@@ -32,8 +32,7 @@
 // 128-replica AO ensemble (1.34 M particles, one launch per class) 4 x 41 us
 // and 4 x 22 us, its whole step 220 and 154 us; the N = 262,144 step kernel
 // (with the integrator) 34 and 24 us; N = 32,768 (four lanes per particle)
-// 14.4 and 11.9 us; N = 30,011 LJ at 3 particles per cell, whole step 46 and
-// 33 us.  Measured equal or slower: the next three runs' table reads in
+// 14.4 and 11.9 us.  Measured equal or slower: the next three runs' table reads in
 // flight during the list stage (39.4 against 39.2 us per step), 5 or 6 waves
 // per SIMD with shorter columns (39.5; 6 waves spill), 64 pairs per round.
 //

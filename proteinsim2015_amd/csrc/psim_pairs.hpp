@@ -14,7 +14,6 @@ namespace psim {
 
 // Positions in the engine's slot-ordered SoA ([3][N]) with one radius.
 struct SoAPos {
-    static constexpr bool kOneRadius = true;
     const double *__restrict__ p;
     int N;
     double radius;
@@ -29,7 +28,6 @@ struct SoAPos {
 // The reference's sortedParticles layout (x,y,z,r per sorted index,
 // systemHandling.cpp:79-83).
 struct AoS4Pos {
-    static constexpr bool kOneRadius = false;
     const double *__restrict__ p;
     __device__ double x(int j) const { return p[4 * (size_t)j]; }
     __device__ double y(int j) const { return p[4 * (size_t)j + 1]; }

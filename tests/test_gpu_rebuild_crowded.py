@@ -94,3 +94,25 @@ def test_ensemble_with_a_crowded_replica():
             assert np.array_equal(together[:g.n], alone)
         first += g.n
     assert np.isfinite(together).all()
+
+
+def test_records_of_a_crowded_box():
+    """The states that the rebuild records for the adjoint, 62 particles per cell
+    (split): gradients with every state recorded are those of the recomputed
+    segments."""
+    n, S, K = 4000, 4, 6
+    g = ps.SystemGeometry(n=n, box=28.0, cells_per_dim=S, cell_size=7.0, integer=False)
+    mods = ps.AOPotential(kT=1.0, well_depth=0.3, cutoff=1.1)
+    integ = ps.BrownianIntegrator(kT=1.0, gamma=1.0, dt=1e-4, seed=5)
+    w = np.random.default_rng(8).standard_normal((n, 3))
+    out = []
+    with ps.GpuSystem(g, mods, integ) as s:
+        s.set_state(ps.rsa_positions(n, g.box, 2))
+        with ps.Adjoint(s, K, 3) as adj:
+            for on in (False, True):
+                adj.set_record_all(on)
+                assert adj.forward() == 0
+                out.append(adj.backward(w, with_gx0=True))
+    assert np.abs(out[0]["gx0"]).max() > 0
+    for k in out[0]:
+        assert np.array_equal(out[0][k], out[1][k]), k
