@@ -26,8 +26,9 @@
 //               were dealt out, and is that of a walk pair by pair.
 //
 // What bounds it: at 0.4 particles per cell (AO, N = 262,144) a wave issues
-// 815 VALU instructions, against 1457 for the cell-by-cell walk, and waits for
-// a chain of about ten loads; VALU issue and the chain share the time.
+// 971 VALU instructions (1,871 with the integrator), against 1,337 for the
+// cell-by-cell walk, and waits for a chain of about ten loads; VALU issue (54 %
+// of the launch) and the chain share the time.
 // Measured on MI355X, the walk first, this second: the pair kernel of the
 // 128-replica AO ensemble (1.34 M particles, one launch per class) 4 x 41 us
 // and 4 x 22 us, its whole step 220 and 154 us; the N = 262,144 step kernel
