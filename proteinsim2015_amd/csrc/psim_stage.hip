@@ -1,7 +1,7 @@
 // psim_stage.hip -- copies between device memory and a caller's pageable
 // arrays through a pinned staging buffer (host code).
 //
-// A pageable hipMemcpy costs, on MI355X boxes, 20 us at 24 KB, 0.35 ms at 0.8 MB
+// A pageable hipMemcpy costs, on MI355X hosts, 20 us at 24 KB, 0.35 ms at 0.8 MB
 // (2.2 GB/s) and 5 ms for 48 MB into fresh pages; the same copies from or to
 // pinned memory take 8 us, 0.02 ms and 0.9 ms, and the host's part (a copy
 // between the staging buffer and the caller's array, page faults included) is
